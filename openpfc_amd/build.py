@@ -44,17 +44,24 @@ def _run(cmd, quiet=True):
 
 
 SOURCES = ["pfc_hip.hip", "variants_common.hip", "variants_f64.hip", "variants_f32.hip",
-           "variants_t_f64.hip", "variants_t_f32.hip", "variants_t_xp.hip", "field_io.hip",
+           "variants_tx_f64.hip", "variants_ty_f64.hip", "variants_tz_f64.hip",
+           "variants_tx_f32.hip", "variants_ty_f32.hip", "variants_tz_f32.hip",
+           "variants_t_xp.hip", "field_io.hip",
            "ensemble.hip"]
 OBJDIR = os.path.join(HERE, "_build")
 
 
 def _stale(obj: str, src: str) -> bool:
-    """Whether obj is older than its source or any header it may include."""
+    """Whether obj is older than its source or any header it includes (the
+    dependency file its compilation wrote; every header without one)."""
     if not os.path.exists(obj):
         return True
     deps = [src] + [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hpp")]
     deps.append(os.path.join(ROOT, "include", "pfc_hip.h"))
+    if os.path.exists(obj + ".d"):
+        with open(obj + ".d") as fh:
+            names = fh.read().replace("\\\n", " ").split()
+        deps = [src] + [f for f in names if os.path.exists(f) and f.startswith(ROOT)]
     t = os.path.getmtime(obj)
     return any(os.path.getmtime(d) > t for d in deps)
 
@@ -72,7 +79,7 @@ def build_library(verbose: bool = False, incremental: bool = False) -> str:
         objs.append(obj)
         if incremental and not _stale(obj, os.path.join(CSRC, src)):
             continue
-        jobs.append([hipcc(), *HIP_FLAGS, "-c", "-o", obj, os.path.join(CSRC, src)])
+        jobs.append([hipcc(), *HIP_FLAGS, "-MD", "-MF", obj + ".d", "-c", "-o", obj, os.path.join(CSRC, src)])
     with ThreadPoolExecutor(max_workers=max(1, min(len(jobs), os.cpu_count() or 4))) as ex:
         list(ex.map(lambda c: _run(c, quiet=not verbose), jobs))
     tmp = LIB + ".tmp"

@@ -23,6 +23,7 @@
 
 #include <cstdint>
 #include <type_traits>
+#include <vector>
 
 namespace pfc_amd {
 
@@ -273,6 +274,12 @@ template <int N_, int E_, int... Rs, bool XP_> struct FftPlan<N_, E_, RadixList<
   }
 };
 
+// Radices of a plan as a host vector.
+template <typename List> struct RadixOf;
+template <int... Rs> struct RadixOf<RadixList<Rs...>> {
+  static std::vector<int> get() { return {Rs...}; }
+};
+
 // LDS view for one line: element pos of this line lives at
 // re[pos*spos + off], im[...] (im plane follows re plane at `plane`).
 template <typename T> struct LdsLine {
@@ -331,8 +338,8 @@ struct Pass {
   // arithmetic type of the butterflies (double for XP plans)
   using C = std::conditional_t<Plan::XP, double, T>;
 
-  __device__ __forceinline__ static void run(cplx<T> (&v)[E], int t,
-                                             const LdsLine<T> &lds,
+  template <typename Lds>
+  __device__ __forceinline__ static void run(cplx<T> (&v)[E], int t, const Lds &lds,
                                              const cplx<T> *__restrict__ tw) {
     // butterflies; element q of butterfly b is v[b + NB*q]
 #pragma unroll
@@ -520,8 +527,8 @@ template <typename T, typename Plan, int DIR, bool SPLIT, bool ROWPAD, bool WAVE
 struct LineFft;
 template <typename T, typename Plan, int DIR, bool SPLIT, bool ROWPAD, bool WAVE, int... Rs>
 struct LineFft<T, Plan, DIR, SPLIT, ROWPAD, WAVE, RadixList<Rs...>> {
-  __device__ __forceinline__ static void run(cplx<T> (&v)[Plan::E], int t,
-                                             const LdsLine<T> &lds,
+  template <typename Lds>
+  __device__ __forceinline__ static void run(cplx<T> (&v)[Plan::E], int t, const Lds &lds,
                                              const cplx<T> *__restrict__ tw) {
     Pass<T, Plan, DIR, SPLIT, ROWPAD, WAVE, 1, 0, Rs...>::run(v, t, lds, tw);
   }

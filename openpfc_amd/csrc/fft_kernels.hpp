@@ -532,16 +532,27 @@ __device__ __forceinline__ void z_mode_ops(const PfcOp &o, const TungOp &p,
 
 // ----------------------------------------------------------------------------
 // Fused step, z pass (natural layout): for L adjacent kx columns at one ky,
-//   ZM_PFC:   A = Fz^-1(opL*Fz(A) + opN*Fz(B))
-//   ZM_TMF:   A = Fz(A); B = Fz^-1(fMF*A)
-//   ZM_TCOMB: A = Fz^-1(expL*A + nW*Fz(B))
+//   ZM_PFC:   out = Fz^-1(opL*Fz(A) + opN*Fz(B))
+//   ZM_TMF:   A = Fz(A); out = Fz^-1(fMF*A)
+//   ZM_TCOMB: out = Fz^-1(expL*A + nW*Fz(B))
 // with the multipliers evaluated per mode on the fly (no tables in HBM).
+//
+// kz enters the multipliers only as kz*kz, and pfc_kc(k) = -pfc_kc(nz - k)
+// exactly, so a column has nz/2 + 1 distinct pairs: the block evaluates those
+// into LDS while its loads are in flight and each mode reads its pair from
+// slot k or nz - k.  A pair costs an exponential and a division in double
+// (about 75 instructions), and on the grids this layout serves each SIMD
+// holds one or two waves, so the evaluations are a serial chain no other wave
+// hides.  Above kZTabMax points the table (16 bytes a pair and column in
+// double) would take the LDS of the blocks that hide latency there, and the
+// pairs are evaluated per element.  Same values and arithmetic either way.
 // ----------------------------------------------------------------------------
 template <typename T> struct PfcZArgs {
   int zero_k0; // mean-split step: the k = 0 mode of the deviation stays 0
   int mode;    // ZMode
   cplx<T> *A;
   cplx<T> *B;
+  cplx<T> *out;
   const cplx<T> *tw;
   PfcOp op;
   TungOp top;
@@ -553,11 +564,18 @@ template <typename T> struct PfcZArgs {
   int ntx;
 };
 
+constexpr int kZTabMax = 256;
+template <typename T, int N, int L> constexpr int z_table_len() {
+  return N <= kZTabMax ? 2 * L * (N / 2 + 1) : 1;
+}
+
 template <typename T, typename Plan, int L, bool SPLIT, int MODE>
 __global__ void __launch_bounds__(L *Plan::TL) k_pfc_z(PfcZArgs<T> a) {
-  constexpr int TL = Plan::TL, E = Plan::E, N = Plan::N;
+  constexpr int TL = Plan::TL, E = Plan::E, N = Plan::N, NH = N / 2 + 1;
   constexpr int NP = row_padded(N);
+  constexpr bool TAB = N <= kZTabMax;
   __shared__ T lds[(SPLIT ? 1 : 2) * L * NP];
+  __shared__ T tab[z_table_len<T, N, L>()]; // [pair member][k][column]
   const int c = threadIdx.x % L, t = threadIdx.x / L;
   const unsigned bid = xcd_block<T, L>(blockIdx.x, gridDim.x);
   const int tx = (int)(bid % (unsigned)a.ntx);
@@ -572,71 +590,69 @@ __global__ void __launch_bounds__(L *Plan::TL) k_pfc_z(PfcZArgs<T> a) {
   PfcOp op = a.op;
   if (a.meps) op.eps = a.meps[b];
   const double kxy = pfc_kxy(op, x, y);
+  auto slot = [&](int e) {
+    const int k = t + TL * e;
+    return (k <= N / 2 ? k : N - k) * L + c;
+  };
 
-  cplx<T> acc[E];
-  if constexpr (MODE == ZM_PFC) {
+  cplx<T> acc[E], v[E];
+  T mul[TAB ? 1 : 2 * E];
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      acc[e] = active ? a.A[base + (long)(t + TL * e) * a.s_pos] : cplx<T>{0, 0};
-    LineFft<T, Plan, -1, SPLIT, true>::run(acc, t, ll, a.tw);
-    T opn[E];
+  for (int e = 0; e < E; ++e) {
+    const long i = base + (long)(t + TL * e) * a.s_pos;
+    acc[e] = active ? (MODE == ZM_TCOMB ? a.B : a.A)[i] : cplx<T>{0, 0};
+    if constexpr (MODE != ZM_TMF)
+      v[e] = active ? (MODE == ZM_TCOMB ? a.A : a.B)[i] : cplx<T>{0, 0};
+  }
+  if constexpr (TAB) {
+    for (int k = t; k < NH; k += TL) {
+      double ma, mb;
+      z_mode_ops<MODE>(op, a.top, kxy, pfc_kc(k, op.nz, op.fz), ma, mb);
+      tab[k * L + c] = (T)ma;
+      if constexpr (MODE != ZM_TMF) tab[NH * L + k * L + c] = (T)mb;
+    }
+    __syncthreads(); // the table is complete
+  } else {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      double l, n;
-      pfc_op_mode(op, kxy, pfc_kc(t + TL * e, op.nz, op.fz), l, n);
-      acc[e] = c_scale(acc[e], (T)l);
-      opn[e] = (T)n;
+      double ma, mb;
+      z_mode_ops<MODE>(op, a.top, kxy, pfc_kc(t + TL * e, op.nz, op.fz), ma, mb);
+      mul[e] = (T)ma;
+      mul[E + e] = (T)mb;
     }
-    {
-      cplx<T> v[E];
+  }
+  auto mul_a = [&](int e) {
+    if constexpr (TAB) return tab[slot(e)];
+    else return mul[e];
+  };
+  auto mul_b = [&](int e) {
+    if constexpr (TAB) return tab[NH * L + slot(e)];
+    else return mul[E + e];
+  };
+  LineFft<T, Plan, -1, SPLIT, true>::run(acc, t, ll, a.tw);
+  if constexpr (MODE == ZM_PFC) {
 #pragma unroll
-      for (int e = 0; e < E; ++e)
-        v[e] = active ? a.B[base + (long)(t + TL * e) * a.s_pos] : cplx<T>{0, 0};
-      LineFft<T, Plan, -1, SPLIT, true>::run(v, t, ll, a.tw);
+    for (int e = 0; e < E; ++e) acc[e] = c_scale(acc[e], mul_a(e));
+    LineFft<T, Plan, -1, SPLIT, true>::run(v, t, ll, a.tw);
 #pragma unroll
-      for (int e = 0; e < E; ++e) acc[e] = c_add(acc[e], c_scale(v[e], opn[e]));
-    }
+    for (int e = 0; e < E; ++e) acc[e] = c_add(acc[e], c_scale(v[e], mul_b(e)));
     if (a.zero_k0 && x == 0 && y == 0 && t == 0) acc[0] = cplx<T>{0, 0};
   } else if constexpr (MODE == ZM_TMF) {
-#pragma unroll
-    for (int e = 0; e < E; ++e)
-      acc[e] = active ? a.A[base + (long)(t + TL * e) * a.s_pos] : cplx<T>{0, 0};
-    LineFft<T, Plan, -1, SPLIT, true>::run(acc, t, ll, a.tw);
     if (active) {
 #pragma unroll
       for (int e = 0; e < E; ++e) a.A[base + (long)(t + TL * e) * a.s_pos] = acc[e];
     }
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      double f, unused;
-      z_mode_ops<ZM_TMF>(op, a.top, kxy, pfc_kc(t + TL * e, op.nz, op.fz), f, unused);
-      acc[e] = c_scale(acc[e], (T)f);
-    }
+    for (int e = 0; e < E; ++e) acc[e] = c_scale(acc[e], mul_a(e));
   } else {
-    // multipliers first, while nothing else is live
-    T opl[E], opn[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      double l, n;
-      z_mode_ops<ZM_TCOMB>(op, a.top, kxy, pfc_kc(t + TL * e, op.nz, op.fz), l, n);
-      opl[e] = (T)l;
-      opn[e] = (T)n;
-    }
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      acc[e] = active ? a.B[base + (long)(t + TL * e) * a.s_pos] : cplx<T>{0, 0};
-    LineFft<T, Plan, -1, SPLIT, true>::run(acc, t, ll, a.tw);
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const cplx<T> h = active ? a.A[base + (long)(t + TL * e) * a.s_pos] : cplx<T>{0, 0};
-      acc[e] = c_add(c_scale(h, opl[e]), c_scale(acc[e], opn[e]));
-    }
+      acc[e] = c_add(c_scale(v[e], mul_a(e)), c_scale(acc[e], mul_b(e)));
   }
   LineFft<T, Plan, +1, SPLIT, true>::run(acc, t, ll, a.tw);
   if (active) {
-    cplx<T> *__restrict__ out = MODE == ZM_TMF ? a.B : a.A;
 #pragma unroll
-    for (int e = 0; e < E; ++e) out[base + (long)(t + TL * e) * a.s_pos] = acc[e];
+    for (int e = 0; e < E; ++e) a.out[base + (long)(t + TL * e) * a.s_pos] = acc[e];
   }
 }
 

@@ -434,14 +434,17 @@ int c2r_impl(pfc_hip_plan_s *p, const void *in, void *out, hipStream_t s,
   return 0;
 }
 
-// z pass of the natural layout on the plan's spectra A and B (ZMode `mode`).
-template <typename T> hipError_t z_natural(pfc_hip_plan_s *p, int mode, hipStream_t s) {
+// z pass of the natural layout (ZMode `mode`): Psi in `in_a`, N or nothing in
+// B, result in `out`.
+template <typename T>
+hipError_t z_natural(pfc_hip_plan_s *p, int mode, void *in_a, void *out, hipStream_t s) {
   const auto &v = pfcz_variants<T>(p->nz)[p->var[ROLE_PFC_Z]];
   PfcZArgs<T> a{};
   a.zero_k0 = (mode == ZM_PFC && p->mean_split) ? 1 : 0;
   a.mode = mode;
-  a.A = (cplx<T> *)p->A;
+  a.A = (cplx<T> *)in_a;
   a.B = (cplx<T> *)p->B;
+  a.out = (cplx<T> *)out;
   a.tw = twp<T>(p, p->nz, v.plan_id);
   a.op = p->op;
   a.top = p->top;
@@ -483,7 +486,7 @@ int step_natural(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev) {
     PFC_HIP_TRY(e, "pfc forward y pass");
   }
   mark(2);
-  PFC_HIP_TRY(z_natural<T>(p, ZM_PFC, s), "pfc z pass");
+  PFC_HIP_TRY(z_natural<T>(p, ZM_PFC, p->A, p->A, s), "pfc z pass");
   mark(3);
   if (p->ny > 1) {
     e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
@@ -647,7 +650,7 @@ int step_tung_natural(pfc_hip_plan_s *p, void *psi, void *mf, hipStream_t s,
     PFC_HIP_TRY(e, "tungsten forward y");
   }
   mark(2);
-  PFC_HIP_TRY(z_natural<T>(p, ZM_TMF, s), "tungsten mean-field z pass");
+  PFC_HIP_TRY(z_natural<T>(p, ZM_TMF, p->A, p->B, s), "tungsten mean-field z pass");
   mark(3);
   if (p->ny > 1) {
     e = col_pass<T>(p, 1, +1, p->B, p->B, nullptr, nullptr, 1, p->P, s);
@@ -673,7 +676,7 @@ int step_tung_natural(pfc_hip_plan_s *p, void *psi, void *mf, hipStream_t s,
     PFC_HIP_TRY(e, "tungsten forward y (N)");
   }
   mark(6);
-  PFC_HIP_TRY(z_natural<T>(p, ZM_TCOMB, s), "tungsten combine z pass");
+  PFC_HIP_TRY(z_natural<T>(p, ZM_TCOMB, p->A, p->A, s), "tungsten combine z pass");
   mark(7);
   if (p->ny > 1) {
     e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);

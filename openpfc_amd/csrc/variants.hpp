@@ -86,6 +86,10 @@ template <typename T> const std::vector<XV<T>> &xc2r_variants(int m);
 template <typename T> const std::vector<PXV<T>> &pfcx_variants(int n);
 template <typename T> const std::vector<TXV<T>> &tungx_variants(int m);
 template <typename T> const std::vector<TV<T>> &t_variants(int kind, int n);
+// the y and z kinds of t_variants (own translation units)
+template <typename T> const std::vector<TV<T>> &ty_fwd_variants(int n);
+template <typename T> const std::vector<TV<T>> &ty_inv_variants(int n);
+template <typename T> const std::vector<TV<T>> &tz_variants(int n);
 #define PFC_AMD_DECLARE_LISTS(T)                                               \
   template <> const std::vector<ColV<T>> &col_variants<T>(int);                \
   template <> const std::vector<ZV<T>> &pfcz_variants<T>(int);                 \
@@ -93,6 +97,9 @@ template <typename T> const std::vector<TV<T>> &t_variants(int kind, int n);
   template <> const std::vector<XV<T>> &xc2r_variants<T>(int);                 \
   template <> const std::vector<PXV<T>> &pfcx_variants<T>(int);               \
   template <> const std::vector<TXV<T>> &tungx_variants<T>(int);               \
+  template <> const std::vector<TV<T>> &ty_fwd_variants<T>(int);               \
+  template <> const std::vector<TV<T>> &ty_inv_variants<T>(int);               \
+  template <> const std::vector<TV<T>> &tz_variants<T>(int);                   \
   template <> const std::vector<TV<T>> &t_variants<T>(int, int);
 PFC_AMD_DECLARE_LISTS(double)
 PFC_AMD_DECLARE_LISTS(float)

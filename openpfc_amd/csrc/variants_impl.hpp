@@ -83,11 +83,6 @@ template <> struct PlansXP<1024> {
                      FftPlan<1024, 4, RadixList<4, 4, 4, 4, 4>, true>>;
 };
 
-template <typename List> struct RadixOf;
-template <int... Rs> struct RadixOf<RadixList<Rs...>> {
-  static std::vector<int> get() { return {Rs...}; }
-};
-
 template <typename Plan> std::string plan_name() {
   std::string s = "r";
   auto r = RadixOf<typename Plan::List>::get();
@@ -173,9 +168,14 @@ void add_col(std::vector<ColV<T>> &v, int pid) {
     v.push_back({plan_name<Plan>() + "/L" + std::to_string(L) + (S ? "/split" : "/full"),
                  pid, &col_launch<T, Plan, L, S>});
 }
+template <typename T, typename Plan, int L, bool S> constexpr bool z_fits() {
+  return col_fits<T, Plan, L, S>() &&
+         ((S ? 1 : 2) * L * row_padded(Plan::N) + z_table_len<T, Plan::N, L>()) * (int)sizeof(T) <=
+             kMaxLds;
+}
 template <typename T, typename Plan, int L, bool S>
 void add_z(std::vector<ZV<T>> &v, int pid) {
-  if constexpr (col_fits<T, Plan, L, S>())
+  if constexpr (z_fits<T, Plan, L, S>())
     v.push_back({plan_name<Plan>() + "/L" + std::to_string(L) + (S ? "/split" : "/full"),
                  pid, &pfcz_launch<T, Plan, L, S>});
 }
@@ -901,17 +901,39 @@ template <int N, int KIND> std::vector<TV<float>> make_t_kind_xp() {
     return empty;                                                              \
   }
 
-#define PFC_AMD_DEFINE_T_LISTS(T)                                              \
+// Transposed-step kinds, one translation unit per group of kinds: the x
+// passes (and the dispatch), the y passes, the z pass.
+#define PFC_AMD_DEFINE_T_X_LISTS(T)                                            \
   template <> const std::vector<TV<T>> &t_variants<T>(int kind, int n) {       \
     static const std::vector<TV<T>> empty;                                     \
-    if (kind < 0 || kind >= TK_COUNT) return empty;                            \
-    PFC_AMD_SWITCH_LEN(n, static const std::vector<TV<T>> v[TK_COUNT] = {      \
-        make_t_kind<T, N_, 0>(), make_t_kind<T, N_, 1>(),                      \
-        make_t_kind<T, N_, 2>(), make_t_kind<T, N_, 3>(),                      \
-        make_t_kind<T, N_, 4>(), make_t_kind<T, N_, 5>(),                      \
-        make_t_kind<T, N_, 6>(), make_t_kind<T, N_, 7>()};                     \
-                          return v[kind];)                                     \
-    return empty;                                                              \
+    switch (kind) {                                                            \
+    case TK_Y_FWD: return ty_fwd_variants<T>(n);                               \
+    case TK_Y_INV: return ty_inv_variants<T>(n);                               \
+    case TK_Z: return tz_variants<T>(n);                                       \
+    case TK_X_FWD: PFC_AMD_T_LIST(T, n, TK_X_FWD)                              \
+    case TK_X_INV: PFC_AMD_T_LIST(T, n, TK_X_INV)                              \
+    case TK_X_R2C: PFC_AMD_T_LIST(T, n, TK_X_R2C)                              \
+    case TK_X_TUNG: PFC_AMD_T_LIST(T, n, TK_X_TUNG)                            \
+    case TK_X_FUSE: PFC_AMD_T_LIST(T, n, TK_X_FUSE)                            \
+    default: return empty;                                                     \
+    }                                                                          \
   }
+#define PFC_AMD_DEFINE_T_Y_LISTS(T)                                            \
+  template <> const std::vector<TV<T>> &ty_fwd_variants<T>(int n) {            \
+    static const std::vector<TV<T>> empty;                                     \
+    PFC_AMD_T_LIST(T, n, TK_Y_FWD)                                             \
+  }                                                                            \
+  template <> const std::vector<TV<T>> &ty_inv_variants<T>(int n) {            \
+    static const std::vector<TV<T>> empty;                                     \
+    PFC_AMD_T_LIST(T, n, TK_Y_INV)                                             \
+  }
+#define PFC_AMD_DEFINE_T_Z_LISTS(T)                                            \
+  template <> const std::vector<TV<T>> &tz_variants<T>(int n) {                \
+    static const std::vector<TV<T>> empty;                                     \
+    PFC_AMD_T_LIST(T, n, TK_Z)                                                 \
+  }
+#define PFC_AMD_T_LIST(T, n, KIND)                                             \
+  PFC_AMD_SWITCH_LEN(n, static const auto v = make_t_kind<T, N_, KIND>(); return v;) \
+  return empty;
 
 } // namespace pfc_amd

@@ -1,0 +1,6 @@
+// Transposed-step variant lists and kernels for double precision: the x passes.
+#include "variants_impl.hpp"
+
+namespace pfc_amd {
+PFC_AMD_DEFINE_T_X_LISTS(double)
+} // namespace pfc_amd

@@ -1,0 +1,6 @@
+// Transposed-step variant lists and kernels for float precision: the y passes.
+#include "variants_impl.hpp"
+
+namespace pfc_amd {
+PFC_AMD_DEFINE_T_Y_LISTS(float)
+} // namespace pfc_amd
