@@ -389,9 +389,14 @@ int pfc_hip_tungsten_operators(pfc_hip_plan_t plan, void *filterMF, void *expL,
  *      boundaries (transposed layout; the autotuner picks 1 when the fused
  *      pass takes under 95% of the time of the two it replaces)
  * The Tungsten step also uses roles 0, 1, 2, 5 (natural) and 8..11
- * (transposed).  Index 0 is the default of each role.  No reference counterpart: the
- * reference delegates shapes to rocFFT; its GPU autotuner only times 1-D
- * block sizes (include/openpfc/runtime/common/gpu_autotune.hpp:295-333).
+ * (transposed).  The last variant of roles 0, 1, 4 and 12 is "plane" where one
+ * z plane of the half spectrum fits a CU's LDS: a block then does the x and the
+ * y pass of a whole plane (role 2 is not used in that direction), and where both
+ * directions of the PFC step are on it a multi-step run makes each step boundary
+ * in one launch, with the bits of single steps.  A new plan starts on "plane"
+ * where that is measured faster, else on index 0 of each role.  No reference
+ * counterpart: the reference delegates shapes to rocFFT; its GPU autotuner only
+ * times 1-D block sizes (include/openpfc/runtime/common/gpu_autotune.hpp:295-333).
  */
 enum {
   PFC_HIP_ROLE_X_R2C = 0,
@@ -423,8 +428,9 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index);
 /*
  * Time every variant of every step role on full steps of psi (`reps` timed
  * steps after one warm-up each; the three fastest of a role are timed twice
- * more, round-robin), keep the fastest per role, then keep the faster step
- * layout.  psi is restored before return (the stream is synchronised).
+ * more, round-robin), keep the fastest per role ("plane" variants by the time of
+ * whole four-step runs against the row kernels tuned before), then keep the
+ * faster step layout.  psi is restored before return (the stream is synchronised).
  * times_ms (may be NULL) receives the fastest time per step of the passes
  * each variant runs, for every variant tried, roles in the order
  * 4, 2, 5, 1, 7, 8, 9, 10, 11, 15 (PFC) or 0, 2, 5, 12, 1, 13, 8, 9, 10, 14, 11

@@ -292,6 +292,25 @@ template <typename T> struct LdsLine {
   }
 };
 
+// LDS view for one line of interleaved complex values (element pos at
+// base[pos*spos + off], moved as one 2-vector: an 8- or 16-byte access instead
+// of two of half the width that hit every other bank).
+template <typename T> struct Vec2;
+template <> struct Vec2<double> { using type = double __attribute__((ext_vector_type(2))); };
+template <> struct Vec2<float> { using type = float __attribute__((ext_vector_type(2))); };
+template <typename T> struct LdsCplx {
+  using V = typename Vec2<T>::type;
+  V *base;
+  int off, spos;
+  __device__ __forceinline__ cplx<T> get(int pos) const {
+    const V v = base[pos * spos + off];
+    return cplx<T>{v.x, v.y};
+  }
+  __device__ __forceinline__ void put(int pos, cplx<T> c) const {
+    base[pos * spos + off] = V{c.x, c.y};
+  }
+};
+
 // LDS padding: one pad position every 16 positions breaks the power-of-two
 // strides of the Stockham write pattern across LDS banks (used by rows and
 // by column tiles, whose L columns are interleaved per position).
@@ -472,6 +491,20 @@ struct Pass {
       else // NS >= 32: q*NS is a multiple of 32
         return d0 + (d0 >> 5) + q * (NS + NS / 32);
     }
+  }
+
+  // Exchange through interleaved storage of the line (unpadded).
+  __device__ __forceinline__ static void exchange(cplx<T> (&v)[E], int t,
+                                                  const LdsCplx<T> &lds) {
+    static_assert(!ROWPAD, "interleaved lines are unpadded");
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int q = 0; q < R; ++q) lds.put(dst_pos(t, b, q), v[b + NB * q]);
+    lds_sync<WAVE>();
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = lds.get(t + TL * e);
+    lds_sync<WAVE>();
   }
 
   __device__ __forceinline__ static void exchange(cplx<T> (&v)[E], int t,

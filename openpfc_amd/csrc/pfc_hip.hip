@@ -3,6 +3,7 @@
 #include "../../include/pfc_hip.h"
 #include "adjoint_kernels.hpp"
 #include "energy_kernels.hpp"
+#include "plane.hpp"
 #include "variants.hpp"
 
 #include <hip/hip_runtime.h>
@@ -119,6 +120,7 @@ struct pfc_hip_plan_s {
   // fused-step state: natural layout (A, B pitched by P) or transposed
   // layouts T1 (A1, B1) and T2 (A2, B2), W*ny*nz complex each
   void *A = nullptr, *B = nullptr;
+  void *C = nullptr; // natural layout with plane kernels: Psi between x/y and z
   void *A1 = nullptr, *B1 = nullptr, *A2 = nullptr, *B2 = nullptr;
   // adjoint workspace: three outbox spectra, two real fields, block partials
   void *adj_lam = nullptr, *adj_P = nullptr, *adj_N = nullptr;
@@ -181,6 +183,11 @@ struct pfc_hip_plan_s {
   // PFC_HIP_FLAG_F64_BUTTERFLIES: single-precision fields whose transposed
   // PFC passes run their butterflies in double (t_variants_xp lists)
   bool xp = false;
+  // the plane kernels take these extents (plane_kernels.hpp)
+  size_t plane_bytes() const {
+    return xp ? 0 : prec == PFC_HIP_F64 ? plane_lds<double>(nx, ny) : plane_lds<float>(nx, ny);
+  }
+  bool plane_ok() const { return plane_bytes() > 0; }
 };
 
 namespace {
@@ -227,6 +234,29 @@ int upload_line_tables(pfc_hip_plan_s *p, int n) {
     p->tw[key] = d;
   }
   return 0;
+}
+
+// exp(-2 pi i k/nx) in double.
+int upload_wn64(pfc_hip_plan_s *p) {
+  if (p->wn64) return 0;
+  const std::vector<long double> w = real_twiddles(p->nx);
+  if (int rc = dalloc(p, &p->wn64, w.size() * sizeof(double), "real twiddles (double)")) return rc;
+  std::vector<double> h(w.begin(), w.end());
+  PFC_HIP_TRY(hipMemcpy(p->wn64, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice),
+              "real twiddles (double)");
+  return 0;
+}
+
+// Twiddles of the plane kernels' column (ny) and row (nx/2) plans.
+int upload_plane_tables(pfc_hip_plan_s *p) {
+  for (int row = 0; row < 2; ++row) {
+    const int n = row ? p->nx / 2 : p->ny;
+    const int pid = p->prec == PFC_HIP_F64 ? plane_pid<double>(row) : plane_pid<float>(row);
+    void *d = nullptr;
+    if (int rc = upload_table(p, &d, line_twiddles(n, pid), "plane twiddles")) return rc;
+    p->tw[std::make_pair(n, pid)] = d;
+  }
+  return p->prec == PFC_HIP_F64 ? 0 : upload_wn64(p);
 }
 
 // Twiddles of the double-butterfly plans of length n: double entries at
@@ -287,7 +317,7 @@ void free_all(pfc_hip_plan_s *p) {
   void **bufs[] = {&p->wn,      &p->work,  &p->A,     &p->B,     &p->A1,
                    &p->B1,      &p->A2,    &p->B2,    &p->adj_lam, &p->adj_P,
                    &p->adj_N,   &p->adj_a, &p->adj_b, &p->adj_part, &p->m_eps,
-                   &p->m_nl,    &p->colmax, &p->wn64};
+                   &p->m_nl,    &p->colmax, &p->wn64, &p->C};
   for (void **b : bufs) {
     if (*b) (void)hipFree(*b);
     *b = nullptr;
@@ -305,19 +335,39 @@ template <typename T> const std::vector<TV<T>> &t_list(const pfc_hip_plan_s *p, 
   return t_variants<T>(kind, n);
 }
 
+// Variants of the roles that own an x pass of the natural layout: the row
+// kernels, then, where the plane kernels take the extents, one more ("plane")
+// that does the y pass of that direction too.
+bool plane_role(int role) {
+  return role == ROLE_X_R2C || role == ROLE_X_C2R || role == ROLE_PFC_X || role == ROLE_X_TUNG;
+}
+template <typename T> int row_variant_count(const pfc_hip_plan_s *p, int role) {
+  const int n = p->role_len(role);
+  switch (role) {
+  case ROLE_X_R2C: return (int)xr2c_variants<T>(n).size();
+  case ROLE_X_C2R: return (int)xc2r_variants<T>(n).size();
+  case ROLE_PFC_X: return (int)pfcx_variants<T>(n).size();
+  case ROLE_X_TUNG: return (int)tungx_variants<T>(n).size();
+  default: return 0;
+  }
+}
+template <typename T> bool on_plane(const pfc_hip_plan_s *p, int role) {
+  return p->plane_ok() && p->var[role] == row_variant_count<T>(p, role);
+}
+
 template <typename T> int variant_count(pfc_hip_plan_s *p, int role) {
   const int n = p->role_len(role);
+  if (plane_role(role)) {
+    const int rows = row_variant_count<T>(p, role);
+    return rows > 0 && p->plane_ok() ? rows + 1 : rows;
+  }
   if (role == ROLE_STEP_LAYOUT) return p->t_ok && !p->xp ? 2 : 1;
   if (role == ROLE_STEP_FUSE)
     return p->t_ok && !t_list<T>(p, TK_X_FUSE, p->role_len(ROLE_T_X_FUSE)).empty() ? 2 : 1;
   if (t_kind_of_role(role) >= 0) return (int)t_list<T>(p, t_kind_of_role(role), n).size();
   switch (role) {
-  case ROLE_X_R2C: return (int)xr2c_variants<T>(n).size();
-  case ROLE_X_C2R: return (int)xc2r_variants<T>(n).size();
   case ROLE_COL_Y: case ROLE_COL_Z: return (int)col_variants<T>(n).size();
-  case ROLE_PFC_X: return (int)pfcx_variants<T>(n).size();
   case ROLE_PFC_Z: return (int)pfcz_variants<T>(n).size();
-  case ROLE_X_TUNG: return (int)tungx_variants<T>(n).size();
   default: return 0;
   }
 }
@@ -325,10 +375,12 @@ template <typename T> int variant_count(pfc_hip_plan_s *p, int role) {
 template <typename T> const std::string *variant_name(pfc_hip_plan_s *p, int role, int v) {
   static const std::string layouts[2] = {"transposed", "natural"};
   static const std::string fuse[2] = {"per_step", "fused"};
+  static const std::string plane = "plane";
   const int n = p->role_len(role);
   if (v < 0 || v >= variant_count<T>(p, role)) return nullptr;
   if (role == ROLE_STEP_LAYOUT) return &layouts[p->t_ok ? v : 1];
   if (role == ROLE_STEP_FUSE) return &fuse[v];
+  if (plane_role(role) && v == row_variant_count<T>(p, role)) return &plane;
   if (t_kind_of_role(role) >= 0) return &t_list<T>(p, t_kind_of_role(role), n)[v].name;
   switch (role) {
   case ROLE_X_R2C: return &xr2c_variants<T>(n)[v].name;
@@ -365,6 +417,27 @@ hipError_t col_pass(pfc_hip_plan_s *p, int axis, int dir, const void *src0,
   return v.fn(dir, a, n_outer, nfields, s);
 }
 
+// Arguments of the plane kernels on spectra of row pitch `pitch`.
+template <typename T> PlaneArgs<T> plane_args(pfc_hip_plan_s *p, int pitch) {
+  PlaneArgs<T> a{};
+  a.nl = nonlin<T>(p);
+  a.mnl = p->members ? (const T *)p->m_nl : nullptr;
+  a.tw_x = twp<T>(p, p->nx / 2, plane_pid<T>(true));
+  a.tw_y = twp<T>(p, p->ny, plane_pid<T>(false));
+  a.wn = (const cplx<double> *)(p->prec == PFC_HIP_F64 ? p->wn : p->wn64);
+  a.nx = p->nx;
+  a.ny = p->ny;
+  a.nz = p->nz;
+  a.pitch = pitch;
+  a.nfields = 1;
+  a.scale = (T)1;
+  return a;
+}
+template <typename T> hipError_t plane_pass(pfc_hip_plan_s *p, int mode, const PlaneArgs<T> &a,
+                                            hipStream_t s) {
+  return plane_launch<T>(mode, a, (long)p->nz * p->batch, s);
+}
+
 template <typename T>
 hipError_t x_c2r_pass(pfc_hip_plan_s *p, const void *in, void *out, int pitch,
                       double scale, hipStream_t s) {
@@ -381,8 +454,16 @@ hipError_t x_c2r_pass(pfc_hip_plan_s *p, const void *in, void *out, int pitch,
   return v.fn(a, s);
 }
 
+// Forward x and y passes of one real field into spectra of row pitch `pitch`.
 template <typename T>
-int r2c_impl(pfc_hip_plan_s *p, const void *in, void *out, hipStream_t s) {
+int r2c_xy(pfc_hip_plan_s *p, const void *in, void *out, int pitch, hipStream_t s) {
+  if (on_plane<T>(p, ROLE_X_R2C)) {
+    PlaneArgs<T> a = plane_args<T>(p, pitch);
+    a.psi_in = (const T *)in;
+    a.dst[0] = (cplx<T> *)out;
+    PFC_HIP_TRY(plane_pass<T>(p, PL_FWD, a, s), "r2c plane pass");
+    return 0;
+  }
   const int m = p->nx / 2;
   const auto &v = xr2c_variants<T>(m)[p->var[ROLE_X_R2C]];
   XArgs<T> a{};
@@ -391,14 +472,40 @@ int r2c_impl(pfc_hip_plan_s *p, const void *in, void *out, hipStream_t s) {
   a.tw = twp<T>(p, m, v.plan_id);
   a.wn = (const cplx<T> *)p->wn;
   a.rows = (long)p->ny * p->nz;
-  a.pitch = p->W;
+  a.pitch = pitch;
   a.scale = (T)1;
-  hipError_t e = v.fn(a, s);
-  PFC_HIP_TRY(e, "r2c x pass");
-  if (p->ny > 1) {
-    e = col_pass<T>(p, 1, -1, out, out, nullptr, nullptr, 1, p->W, s);
-    PFC_HIP_TRY(e, "r2c y pass");
+  PFC_HIP_TRY(v.fn(a, s), "r2c x pass");
+  if (p->ny > 1)
+    PFC_HIP_TRY(col_pass<T>(p, 1, -1, out, out, nullptr, nullptr, 1, pitch, s), "r2c y pass");
+  return 0;
+}
+
+// Inverse y and x passes of `in` (row pitch `pitch`) into a real field times
+// `scale`; the y pass goes through `work` (which may be `in`) off the plane
+// kernels.
+template <typename T>
+int c2r_yx(pfc_hip_plan_s *p, const void *in, void *work, void *out, int pitch, double scale,
+           hipStream_t s) {
+  if (on_plane<T>(p, ROLE_X_C2R)) {
+    PlaneArgs<T> a = plane_args<T>(p, pitch);
+    a.src = (const cplx<T> *)in;
+    a.psi_out = (T *)out;
+    a.scale = (T)scale;
+    PFC_HIP_TRY(plane_pass<T>(p, PL_INV, a, s), "c2r plane pass");
+    return 0;
   }
+  if (p->ny > 1) {
+    PFC_HIP_TRY(col_pass<T>(p, 1, +1, in, work, nullptr, nullptr, 1, pitch, s), "c2r y pass");
+    in = work;
+  }
+  PFC_HIP_TRY(x_c2r_pass<T>(p, in, out, pitch, scale, s), "c2r x pass");
+  return 0;
+}
+
+template <typename T>
+int r2c_impl(pfc_hip_plan_s *p, const void *in, void *out, hipStream_t s) {
+  hipError_t e;
+  if (int rc = r2c_xy<T>(p, in, out, p->W, s)) return rc;
   if (p->nz > 1) {
     e = col_pass<T>(p, 2, -1, out, out, nullptr, nullptr, 1, p->W, s);
     PFC_HIP_TRY(e, "r2c z pass");
@@ -423,15 +530,8 @@ int c2r_impl(pfc_hip_plan_s *p, const void *in, void *out, hipStream_t s,
     PFC_HIP_TRY(e, "c2r z pass");
     cur = work;
   }
-  if (p->ny > 1) {
-    e = col_pass<T>(p, 1, +1, cur, work, nullptr, nullptr, 1, p->W, s);
-    PFC_HIP_TRY(e, "c2r y pass");
-    cur = work;
-  }
-  e = x_c2r_pass<T>(p, cur, out, p->W,
-                    1.0 / ((double)p->nx * (double)p->ny * (double)p->nz), s);
-  PFC_HIP_TRY(e, "c2r x pass");
-  return 0;
+  return c2r_yx<T>(p, cur, work, out, p->W,
+                   1.0 / ((double)p->nx * (double)p->ny * (double)p->nz), s);
 }
 
 // z pass of the natural layout (ZMode `mode`): Psi in `in_a`, N or nothing in
@@ -456,8 +556,29 @@ hipError_t z_natural(pfc_hip_plan_s *p, int mode, void *in_a, void *out, hipStre
   return v.fn(a, (long)p->ny * p->batch, s);
 }
 
-// One fused PFC step: 5 launches.  `ev` (optional) receives 6 events
-// bracketing the 5 passes.
+// Spectrum that holds Psi between the x/y passes and the z pass of the natural
+// layout: the plane kernels leave it in C (a boundary's two blocks of a plane
+// both read A), the row kernels in A.
+template <typename T> void *natural_psi(pfc_hip_plan_s *p) {
+  return on_plane<T>(p, ROLE_PFC_X) ? p->C : p->A;
+}
+
+// Plane pass that ends in Psi and N before the z pass: from psi (PL_FWD), or
+// from the spectrum the z pass left in A (PL_BND).
+template <typename T>
+hipError_t plane_fwd(pfc_hip_plan_s *p, int mode, const void *psi, hipStream_t s) {
+  PlaneArgs<T> a = plane_args<T>(p, p->P);
+  a.psi_in = (const T *)psi;
+  a.src = (const cplx<T> *)p->A;
+  a.dst[0] = (cplx<T> *)p->C;
+  a.dst[1] = (cplx<T> *)p->B;
+  a.nfields = 2;
+  return plane_pass<T>(p, mode, a, s);
+}
+
+// One fused PFC step: 5 launches, 4 or 3 with plane kernels.  `ev` (optional)
+// receives 6 events bracketing the 5 passes (a plane pass counts as its x
+// pass; the y pass it includes takes no time).
 template <typename T>
 int step_natural(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev) {
   hipError_t e;
@@ -465,7 +586,10 @@ int step_natural(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev) {
     if (ev) (void)hipEventRecord(ev[i], s);
   };
   mark(0);
-  {
+  if (on_plane<T>(p, ROLE_PFC_X)) {
+    PFC_HIP_TRY(plane_fwd<T>(p, PL_FWD, psi, s), "pfc forward plane pass");
+    mark(1);
+  } else {
     const auto &v = pfcx_variants<T>(p->nx)[p->var[ROLE_PFC_X]];
     PfcXArgs<T> a{};
     a.nl = nonlin<T>(p);
@@ -479,25 +603,48 @@ int step_natural(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev) {
     a.pitch = p->P;
     e = v.fn(a, s);
     PFC_HIP_TRY(e, "pfc forward x pass");
-  }
-  mark(1);
-  if (p->ny > 1) {
-    e = col_pass<T>(p, 1, -1, p->A, p->A, p->B, p->B, 2, p->P, s);
-    PFC_HIP_TRY(e, "pfc forward y pass");
+    mark(1);
+    if (p->ny > 1) {
+      e = col_pass<T>(p, 1, -1, p->A, p->A, p->B, p->B, 2, p->P, s);
+      PFC_HIP_TRY(e, "pfc forward y pass");
+    }
   }
   mark(2);
-  PFC_HIP_TRY(z_natural<T>(p, ZM_PFC, p->A, p->A, s), "pfc z pass");
+  PFC_HIP_TRY(z_natural<T>(p, ZM_PFC, natural_psi<T>(p), p->A, s), "pfc z pass");
   mark(3);
-  if (p->ny > 1) {
-    e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
-    PFC_HIP_TRY(e, "pfc inverse y pass");
+  if (on_plane<T>(p, ROLE_X_C2R)) {
+    mark(4);
+    // 1/(nx ny nz) is folded into opL/opN
+    if (int rc = c2r_yx<T>(p, p->A, p->A, psi, p->P, 1.0, s)) return rc;
+  } else {
+    if (p->ny > 1) {
+      e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
+      PFC_HIP_TRY(e, "pfc inverse y pass");
+    }
+    mark(4);
+    e = x_c2r_pass<T>(p, p->A, psi, p->P, 1.0, s);
+    PFC_HIP_TRY(e, "pfc inverse x pass");
   }
-  mark(4);
-  // 1/(nx ny nz) is folded into opL/opN
-  e = x_c2r_pass<T>(p, p->A, psi, p->P, 1.0, s);
-  PFC_HIP_TRY(e, "pfc inverse x pass");
   mark(5);
   return 0;
+}
+
+// Whether multi-step PFC runs keep psi on chip between steps with the plane
+// kernels: one boundary pass (PL_BND) per step boundary, the arithmetic of
+// PL_INV and PL_FWD, so that a run gives the bits of its single steps.
+template <typename T> bool plane_steps(pfc_hip_plan_s *p) {
+  return !p->transposed() && !p->tungsten() && on_plane<T>(p, ROLE_PFC_X) &&
+         on_plane<T>(p, ROLE_X_C2R);
+}
+
+// nsteps >= 1 PFC steps of the natural layout on the plane kernels:
+// 2*nsteps + 1 launches.
+template <typename T> int steps_plane(pfc_hip_plan_s *p, void *psi, int nsteps, hipStream_t s) {
+  for (int i = 0; i < nsteps; ++i) {
+    PFC_HIP_TRY(plane_fwd<T>(p, i == 0 ? PL_FWD : PL_BND, psi, s), "pfc plane pass");
+    PFC_HIP_TRY(z_natural<T>(p, ZM_PFC, natural_psi<T>(p), p->A, s), "pfc z pass");
+  }
+  return c2r_yx<T>(p, p->A, p->A, psi, p->P, 1.0, s);
 }
 
 // Step buffers of the active layout (allocated on first use).
@@ -513,6 +660,9 @@ int step_buffers(pfc_hip_plan_s *p) {
     const size_t c = p->padded() * 2 * p->esize * p->batch;
     if (!rc) rc = dalloc(p, &p->A, c, "step spectrum A");
     if (!rc) rc = dalloc(p, &p->B, c, "step spectrum B");
+    const bool plane = p->prec == PFC_HIP_F64 ? on_plane<double>(p, ROLE_PFC_X)
+                                              : on_plane<float>(p, ROLE_PFC_X);
+    if (!rc && plane && !p->tungsten()) rc = dalloc(p, &p->C, c, "step spectrum C");
   }
   return rc;
 }
@@ -631,8 +781,13 @@ int step_tung_natural(pfc_hip_plan_s *p, void *psi, void *mf, hipStream_t s,
   const int m = p->nx / 2;
   const long rows = (long)p->ny * p->nz;
   hipError_t e;
+  // a plane pass does the x pass of its slot and the y pass next to it
+  const bool pf = on_plane<T>(p, ROLE_X_R2C), pm = on_plane<T>(p, ROLE_X_TUNG),
+             pi = on_plane<T>(p, ROLE_X_C2R);
   mark(0);
-  {
+  if (pf) {
+    if (int rc = r2c_xy<T>(p, psi, p->A, p->P, s)) return rc;
+  } else {
     const auto &v = xr2c_variants<T>(m)[p->var[ROLE_X_R2C]];
     XArgs<T> a{};
     a.in = (const T *)psi;
@@ -645,19 +800,27 @@ int step_tung_natural(pfc_hip_plan_s *p, void *psi, void *mf, hipStream_t s,
     PFC_HIP_TRY(v.fn(a, s), "tungsten forward x");
   }
   mark(1);
-  if (p->ny > 1) {
+  if (!pf && p->ny > 1) {
     e = col_pass<T>(p, 1, -1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
     PFC_HIP_TRY(e, "tungsten forward y");
   }
   mark(2);
   PFC_HIP_TRY(z_natural<T>(p, ZM_TMF, p->A, p->B, s), "tungsten mean-field z pass");
   mark(3);
-  if (p->ny > 1) {
+  if (!pm && p->ny > 1) {
     e = col_pass<T>(p, 1, +1, p->B, p->B, nullptr, nullptr, 1, p->P, s);
     PFC_HIP_TRY(e, "tungsten mean-field inverse y");
   }
   mark(4);
-  {
+  if (pm) {
+    PlaneArgs<T> a = plane_args<T>(p, p->P);
+    a.tnl = tung_nonlin<T>(p);
+    a.psi_in = (const T *)psi;
+    a.mf_out = (T *)mf;
+    a.src = (const cplx<T> *)p->B;
+    a.dst[0] = (cplx<T> *)p->B;
+    PFC_HIP_TRY(plane_pass<T>(p, PL_TUNG, a, s), "tungsten plane pass");
+  } else {
     const auto &v = tungx_variants<T>(m)[p->var[ROLE_X_TUNG]];
     TungXArgs<T> a{};
     a.nl = tung_nonlin<T>(p);
@@ -671,19 +834,24 @@ int step_tung_natural(pfc_hip_plan_s *p, void *psi, void *mf, hipStream_t s,
     PFC_HIP_TRY(v.fn(a, s), "tungsten fused x pass");
   }
   mark(5);
-  if (p->ny > 1) {
+  if (!pm && p->ny > 1) {
     e = col_pass<T>(p, 1, -1, p->B, p->B, nullptr, nullptr, 1, p->P, s);
     PFC_HIP_TRY(e, "tungsten forward y (N)");
   }
   mark(6);
   PFC_HIP_TRY(z_natural<T>(p, ZM_TCOMB, p->A, p->A, s), "tungsten combine z pass");
   mark(7);
-  if (p->ny > 1) {
-    e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
-    PFC_HIP_TRY(e, "tungsten inverse y");
+  if (pi) {
+    mark(8);
+    if (int rc = c2r_yx<T>(p, p->A, p->A, psi, p->P, 1.0, s)) return rc;
+  } else {
+    if (p->ny > 1) {
+      e = col_pass<T>(p, 1, +1, p->A, p->A, nullptr, nullptr, 1, p->P, s);
+      PFC_HIP_TRY(e, "tungsten inverse y");
+    }
+    mark(8);
+    PFC_HIP_TRY(x_c2r_pass<T>(p, p->A, psi, p->P, 1.0, s), "tungsten inverse x");
   }
-  mark(8);
-  PFC_HIP_TRY(x_c2r_pass<T>(p, p->A, psi, p->P, 1.0, s), "tungsten inverse x");
   mark(9);
   return 0;
 }
@@ -909,6 +1077,34 @@ __global__ void __launch_bounds__(256) k_stream_copy(const uint4 *__restrict__ s
   if (i < n) dst[i] = src[i];
 }
 
+// Whether the plane kernels are the default of the x roles.  One block takes a
+// plane, so they need planes enough to keep the CUs busy and lose where few
+// large ones leave most of the chip idle.  Measured (us, plane against row and
+// column kernels; run = step of a multi-step run, one = single step):
+//   FP64 32x32x32    run 11.6 / 19.0  one 17.0 / 23.2  r2c 15.0 / 17.1
+//   FP64 64x64x64    run 15.9 / 23.6  one 20.4 / 24.1  r2c 14.4 / 16.6
+//   FP64 128x128x128 run 43.0 / 60.6  one 50.0 / 59.5  r2c 32.3 / 42.7
+//   FP32 96x96x96    run 26.6 / 36.1  one 32.2 / 36.4  r2c 17.6 / 21.5
+//   FP32 96x96x512   run 66.5 / 85.5  one 73.1 / 85.7  r2c 36.5 / 50.0
+//   FP32 256x64x64   run 25.4 / 33.7  one 33.8 / 33.2  r2c 19.5 / 21.0
+//   FP32 192x96x48   run 29.4 / 35.6  one 37.9 / 35.7  r2c 21.0 / 22.4
+//   FP64 128x128x32  run 31.1 / 32.5  one 38.6 / 32.1  r2c 21.3 / 19.3
+//   FP64 192x48x24   run 22.8 / 27.0  one 28.5 / 27.3  r2c 16.1 / 18.1
+// so: from 64 planes on, or where a plane's bytes are at most 1600 per plane
+// there is.  Above 140 KB (FP32 192x192: 149 KB) a CU holds one block and the
+// column passes are as fast (run 96.8 / 96.0, one 103 / 94.6 us at 192^3).
+bool plane_variant_default(const pfc_hip_plan_s *p) {
+  const size_t b = p->plane_bytes();
+  return b > 0 && b <= 140 * 1024 && (p->nz >= 64 || b <= (size_t)1600 * p->nz);
+}
+
+// The variant each role of a new plan starts with.
+template <typename T> void default_variants(pfc_hip_plan_s *p) {
+  for (int r = 0; r < ROLE_COUNT; ++r)
+    if (plane_role(r) && row_variant_count<T>(p, r) > 0 && plane_variant_default(p))
+      p->var[r] = row_variant_count<T>(p, r);
+}
+
 int check_plan(pfc_hip_plan_t p) {
   if (!p) return fail(PFC_HIP_EINVAL, "null plan");
   return 0;
@@ -983,6 +1179,14 @@ int pfc_hip_plan_create(int nx, int ny, int nz, int precision, int flags,
   if (!rc) rc = upload_line_tables(p, ny);
   if (!rc) rc = upload_line_tables(p, nz);
   if (!rc) rc = upload_table(p, &p->wn, real_twiddles(nx), "real twiddles");
+  if (!rc && p->plane_ok()) {
+    rc = upload_plane_tables(p);
+    if (!rc) {
+      const hipError_t e = precision == PFC_HIP_F64 ? plane_init<double>() : plane_init<float>();
+      if (e != hipSuccess)
+        rc = fail(PFC_HIP_EDEVICE, std::string("plane kernels: ") + hipGetErrorString(e));
+    }
+  }
   if (!rc) {
     bool ok = true;
     for (int r = 0; r < ROLE_COUNT; ++r) {
@@ -1008,24 +1212,17 @@ int pfc_hip_plan_create(int nx, int ny, int nz, int precision, int flags,
     }
     for (int n : {nx, nx / 2, ny, nz})
       if (!rc) rc = upload_line_tables_xp(p, n);
-    if (!rc) {
-      const std::vector<long double> w = real_twiddles(nx);
-      rc = dalloc(p, &p->wn64, w.size() * sizeof(double), "real twiddles (double)");
-      if (!rc) {
-        std::vector<double> h(w.begin(), w.end());
-        hipError_t e = hipMemcpy(p->wn64, h.data(), h.size() * sizeof(double),
-                                 hipMemcpyHostToDevice);
-        if (e != hipSuccess)
-          rc = fail(PFC_HIP_EDEVICE, std::string("real twiddles (double): ") +
-                                         hipGetErrorString(e));
-      }
-    }
+    if (!rc) rc = upload_wn64(p);
   }
   if (rc) {
     free_all(p);
     delete p;
     return rc;
   }
+  if (precision == PFC_HIP_F64)
+    default_variants<double>(p);
+  else
+    default_variants<float>(p);
   *plan = p;
   return 0;
 }
@@ -1233,6 +1430,11 @@ int pfc_hip_pfc_step(pfc_hip_plan_t plan, void *psi, int nsteps, void *stream) {
       if (int rc = step_buffers(plan)) return rc;
       return f64 ? steps_fused<double>(plan, psi, nsteps, s, nullptr)
                  : steps_fused<float>(plan, psi, nsteps, s, nullptr);
+    }
+    if (f64 ? plane_steps<double>(plan) : plane_steps<float>(plan)) {
+      if (int rc = step_buffers(plan)) return rc;
+      return f64 ? steps_plane<double>(plan, psi, nsteps, s)
+                 : steps_plane<float>(plan, psi, nsteps, s);
     }
   }
   for (int i = 0; i < nsteps; ++i) {
@@ -1701,7 +1903,7 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index) {
     if (int rc = set_device(plan)) return rc;
     (void)hipDeviceSynchronize();
     void **drop[4] = {&plan->A1, &plan->B1, &plan->A2, &plan->B2};
-    void **drop_nat[2] = {&plan->A, &plan->B};
+    void **drop_nat[3] = {&plan->A, &plan->B, &plan->C};
     const size_t tb = plan->outbox() * 2 * plan->esize;
     const size_t nb = plan->padded() * 2 * plan->esize * plan->batch;
     if (index == 1) {
@@ -1714,7 +1916,8 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index) {
   }
   if (plan->var[role] != index) ++plan->gen;
   plan->var[role] = index;
-  if (role == ROLE_STEP_LAYOUT && plan->ops_ready) return step_buffers(plan);
+  if ((role == ROLE_STEP_LAYOUT || plane_role(role)) && plan->ops_ready)
+    return step_buffers(plan);
   return 0;
 }
 
@@ -1779,6 +1982,10 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
       if (passes & (1u << k)) t += pm[k];
     return t;
   };
+  auto row_variants = [&](int role) {
+    return plan->prec == PFC_HIP_F64 ? row_variant_count<double>(plan, role)
+                                     : row_variant_count<float>(plan, role);
+  };
   int slot = 0;
   double layout_ms[2] = {0, 0};
   double role_best[ROLE_COUNT];
@@ -1790,11 +1997,24 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
   for (int li = 0; li < layouts && !rc; ++li) {
     const int layout = two ? 1 - li : (plan->t_ok ? 0 : 1);
     rc = pfc_hip_variant_set(plan, ROLE_STEP_LAYOUT, two ? layout : 0);
+    // the row kernels of the natural layout are tuned first (with the y passes
+    // they need), the plane kernels set against them below
+    int plane_slot[ROLE_COUNT];
+    for (int &ps : plane_slot) ps = -1;
+    for (int si = 0; si < nspans; ++si)
+      if (spans[si].layout == layout && plane_role(spans[si].role) &&
+          plan->var[spans[si].role] >= row_variants(spans[si].role))
+        plan->var[spans[si].role] = 0;
     for (int si = 0; si < nspans && !rc; ++si) {
       const RoleSpan &sp = spans[si];
       if (sp.layout != layout) continue;
       int count = 0;
       pfc_hip_variant_count(plan, sp.role, &count);
+      if (plane_role(sp.role) && count > row_variants(sp.role)) {
+        --count;
+        plane_slot[sp.role] = slot + count;
+        if (times_ms && slot + count < max_times) times_ms[slot + count] = 0.0;
+      }
       // Each variant is scored by its fastest rep (interference only adds
       // time); the kTop best are then timed again, round-robin, so that a
       // drift of the clock over the sweep cannot decide between close ones.
@@ -1828,7 +2048,54 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
       }
       plan->var[sp.role] = best_v;
       role_best[sp.role] = best;
-      slot += count;
+      slot += count + (plane_slot[sp.role] >= 0 ? 1 : 0);
+    }
+    // The plane kernels against the tuned row and column kernels, by the time
+    // of whole multi-step runs (PFC runs fuse the step boundary when both
+    // directions are on them, which no single pass shows): the best of every
+    // combination over the roles, starting from all on.
+    std::vector<int> pr, row_best;
+    for (int si = 0; si < nspans; ++si)
+      if (spans[si].layout == layout && plane_slot[spans[si].role] >= 0) {
+        pr.push_back(spans[si].role);
+        row_best.push_back(plan->var[spans[si].role]);
+      }
+    if (!rc && !pr.empty()) {
+      constexpr int kRun = 4;
+      double best = 1e300;
+      unsigned best_mask = 0;
+      auto apply = [&](unsigned mask) {
+        for (size_t i = 0; i < pr.size(); ++i)
+          plan->var[pr[i]] = (mask >> i & 1) ? row_variants(pr[i]) : row_best[i];
+      };
+      for (unsigned m = 1u << pr.size(); m-- > 0 && !rc;) {
+        apply(m);
+        double t = 1e300;
+        for (int r = 0; r <= reps && !rc; ++r) {
+          float ms = 0;
+          hipError_t he = hipEventRecord(ev[0], s);
+          if (he == hipSuccess) rc = pfc_hip_pfc_step(plan, psi, kRun, s);
+          if (rc) break;
+          if (he == hipSuccess) he = hipEventRecord(ev[1], s);
+          if (he == hipSuccess) he = hipEventSynchronize(ev[1]);
+          if (he == hipSuccess) he = hipEventElapsedTime(&ms, ev[0], ev[1]);
+          if (he != hipSuccess) {
+            rc = fail(PFC_HIP_EDEVICE, std::string("autotune run: ") + hipGetErrorString(he));
+            break;
+          }
+          if (r > 0) t = std::min(t, (double)ms / kRun);
+        }
+        for (size_t i = 0; i < pr.size(); ++i) // reported: the fastest step with the role on
+          if ((m >> i & 1) && times_ms && plane_slot[pr[i]] < max_times) {
+            double &w = times_ms[plane_slot[pr[i]]];
+            w = w > 0 ? std::min(w, t) : t;
+          }
+        if (t < best) {
+          best = t;
+          best_mask = m;
+        }
+      }
+      apply(best_mask);
     }
     if (!rc && layout == 0 && !plan->tungsten()) {
       // the fused step boundary of multi-step runs, timed on its own: each

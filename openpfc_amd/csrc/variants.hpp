@@ -109,6 +109,12 @@ PFC_AMD_DECLARE_LISTS(float)
 // Plan ids from kXpPid on are the double-butterfly plans (their tables hold
 // double entries whatever the field precision).
 constexpr int kXpPid = 64;
+// The plane kernels' line plans: columns at plane_pid<T>(false), rows at
+// plane_pid<T>(true).
+constexpr int kPlanePid = 128;
+template <typename T> constexpr int plane_pid(bool row) {
+  return kPlanePid + (sizeof(T) == 8 ? 0 : 2) + (row ? 1 : 0);
+}
 std::vector<int> radices_for(int n, int plan_id);
 int plan_count(int n);
 int plan_count_xp(int n);

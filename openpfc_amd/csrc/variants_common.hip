@@ -1,4 +1,5 @@
 // Precision-independent plan queries.
+#include "plane.hpp"
 #include "variants_impl.hpp"
 
 namespace pfc_amd {
@@ -27,6 +28,10 @@ int plan_count_xp(int n) {
 }
 
 std::vector<int> radices_for(int n, int pid) {
+  if (pid == plane_pid<double>(false)) return plane_radices<double, false>(n);
+  if (pid == plane_pid<double>(true)) return plane_radices<double, true>(n);
+  if (pid == plane_pid<float>(false)) return plane_radices<float, false>(n);
+  if (pid == plane_pid<float>(true)) return plane_radices<float, true>(n);
   if (pid >= kXpPid) {
     PFC_AMD_SWITCH_LEN(n, return radices_in(typename PlansXP<N_>::L{}, pid - kXpPid);)
     return {};
