@@ -84,7 +84,8 @@ NT_KERNELS = ("k_tz", "k_tx_inv", "k_tx_fwd_w", "k_ty_fwd_w", "k_ty_inv_w")
 
 def variant_key(kernel, prec, n, variant, direction=None, mode=0):
     """rocprof short name (openpfc_amd.profile_summary.short_name) of a variant;
-    `mode` is the z-pass kind (0 PFC, 1 Tungsten mean field, 2 Tungsten combine)."""
+    `mode` is the z-pass kind (0 PFC, 1 Tungsten mean field, 2 Tungsten combine,
+    3 PFC with the kept spectrum)."""
     import re
     t = "double" if prec == "f64" else "float"
     if kernel == "k_tx_fuse":  # "rA/EA+rB/EB/G8/split[/wN]": nx/2- and nx-point plans
@@ -94,6 +95,11 @@ def variant_key(kernel, prec, n, variant, direction=None, mode=0):
         wpe = pb[4][1:] if len(pb) > 4 and pb[4][:1] == "w" else "1"  # waves per SIMD cap
         return (f"k_tx_fuse<{t},N{n // 2}/E{ea[1:]},r{ra[1:]}+N{n}/E{pb[1][1:]},r{pb[0][1:]},"
                 f"{pb[2][1:]},{'true' if pb[3] == 'split' else 'false'},{wpe}>")
+    if kernel == "k_tx_bnd":  # "rA/EA/G8[/wN][/nt]": the nx/2-point plan, both directions
+        parts = variant.split("/")
+        wpe = [p[1:] for p in parts if p[:1] == "w"] or ["1"]
+        return (f"k_tx_bnd<{t},N{n // 2}/E{parts[1][1:]},r{parts[0][1:]},{parts[2][1:]},{wpe[0]},"
+                f"{'true' if 'nt' in parts else 'false'}>")
     parts = variant.split("/")
     nt = "nt" in parts  # non-temporal lines: the kernel's last template argument
     xp = "xp" in parts  # a plan with double butterflies
@@ -155,9 +161,10 @@ def pass_bytes(n: int, esize: int):
 
 def fused_pass_bytes(n: int, esize: int):
     """Algorithmic bytes per launch of the steady-state passes of a fused
-    multi-step run: y forward 4C, z 3C, y inverse 2C, fused boundary C + 2C."""
+    multi-step run, which keeps Psi's spectrum between steps and transforms only
+    N: y forward 2C, z 2C + 2C, y inverse 2C, boundary C + C."""
     C = 2 * esize * (n // 2 + 1) * n * n
-    return {"y_fwd": 4 * C, "z_fused": 3 * C, "y_inv": 2 * C, "x_boundary_fused": 3 * C}
+    return {"y_fwd": 2 * C, "z_fused": 4 * C, "y_inv": 2 * C, "x_boundary_fused": 2 * C}
 
 
 def tung_pass_bytes(n: int, esize: int):
@@ -865,7 +872,7 @@ def main(argv=None):
         achieved = fb[dname] / (fk[dname] * 1e-3)
         kern, role = {"y_fwd": ("k_ty_fwd", "t_y_fwd"), "z_fused": ("k_tz", "t_z"),
                       "y_inv": ("k_ty_inv", "t_y_inv"),
-                      "x_boundary_fused": ("k_tx_fuse", "t_x_fuse")}[dname]
+                      "x_boundary_fused": ("k_tx_bnd", "t_x_fuse")}[dname]
         alg_launch = fb[dname]
         run_bytes = sum(fb.values()) + 2 * 8 * n ** 3 / args.steps
     else:
@@ -876,7 +883,7 @@ def main(argv=None):
         alg_launch = pb[dname]
         run_bytes = step_bytes
     kkey = variant_key(kern, "f64", n, chosen64[role],
-                       direction=(-1 if dname == "y_fwd" else 1))
+                       direction=(-1 if dname == "y_fwd" else 1), mode=3 if fused else 0)
     traffic = None
     tpath = args.traffic or os.path.join(ROOT, "profiles", f"traffic_pfc_step_{n}_f64.json")
     if os.path.exists(tpath):

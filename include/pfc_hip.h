@@ -161,12 +161,14 @@ int pfc_hip_pfc_set_operators(pfc_hip_plan_t plan, int model_kind,
  * steps: psi_hat <- opL*F(psi) + opN*F(psi^3); psi <- F^-1(psi_hat).
  * Replaces PFCModel::step (10_complete_pfc_model.cpp:121-144) called
  * nsteps times.  Requires pfc_hip_pfc_set_operators.  With nsteps >= 2 in
- * the transposed layout and role 16 set to 1, the inverse x pass of each
- * step and the forward x pass of the next run as one fused pass that keeps
- * psi on chip (role 15), so psi is written once at the end: 2R fewer bytes
- * per step boundary.  The fused pass may pair different transform plans
- * than the two passes it replaces, so such a call agrees with repeated
- * single steps to rounding, not bit for bit.
+ * the transposed layout and role 16 at 1 (its default there), the call keeps
+ * psi's spectrum between its steps: only the nonlinearity is transformed
+ * forward, psi exists on chip alone at a step boundary (role 15) and is
+ * written once at the end, and a step moves 10 half spectra instead of 12 and
+ * two real fields.  Such a call agrees with repeated single steps to rounding,
+ * not bit for bit: psi is not rounded through real space.  Set role 16 to 0
+ * where a run has to be the same however it is cut into calls.  (Every so many
+ * steps, at most 64, the spectrum is made anew from psi.)
  */
 int pfc_hip_pfc_step(pfc_hip_plan_t plan, void *psi, int nsteps, void *stream);
 
@@ -257,7 +259,8 @@ int pfc_hip_pfc_set_members(pfc_hip_plan_t plan, const double *eps, const double
  * boundaries: the launches of that fused run, kernel_ms[0] the forward x of
  * the first step, 1..3 the mean y, z and inverse y passes, 4 the inverse x of
  * the last step and 5 the mean fused boundary pass (otherwise kernel_ms[5]
- * = 0).  No reference counterpart (profiling aid).
+ * = 0).  The means are over the steps after the first, which alone transforms
+ * psi too.  No reference counterpart (profiling aid).
  */
 int pfc_hip_pfc_step_timed(pfc_hip_plan_t plan, void *psi, int nsteps,
                            void *stream, double *kernel_ms, int nkernels);
@@ -383,18 +386,18 @@ int pfc_hip_tungsten_operators(pfc_hip_plan_t plan, void *filterMF, void *expL,
  *   12 natural Tungsten step: fused x pass (inverse, N, forward)
  *   13 transposed Tungsten step: forward x of psi
  *   14 transposed Tungsten step: fused x pass
- *   15 transposed PFC multi-step runs: fused step boundary (inverse x of a
- *      step with the forward x of the next)
- *   16 multi-step runs: 0 as single steps (default), 1 with fused step
- *      boundaries (transposed layout; the autotuner picks 1 when the fused
- *      pass takes under 95% of the time of the two it replaces)
+ *   15 transposed PFC multi-step runs: step boundary (inverse x of a step,
+ *      nonlinearity, forward x of it)
+ *   16 multi-step runs: 0 as single steps, 1 with the kept spectrum and fused
+ *      step boundaries (transposed layout, the default there; the autotuner
+ *      keeps the faster of the two by the time of whole runs)
  * The Tungsten step also uses roles 0, 1, 2, 5 (natural) and 8..11
  * (transposed).  The last variant of roles 0, 1, 4 and 12 is "plane" where one
  * z plane of the half spectrum fits a CU's LDS: a block then does the x and the
  * y pass of a whole plane (role 2 is not used in that direction), and where both
  * directions of the PFC step are on it a multi-step run makes each step boundary
  * in one launch, with the bits of single steps.  A new plan starts on "plane"
- * where that is measured faster, else on index 0 of each role.  No reference
+ * where that is measured faster, and on index 0 of the other roles but 16.  No reference
  * counterpart: the reference delegates shapes to rocFFT; its GPU autotuner only
  * times 1-D block sizes (include/openpfc/runtime/common/gpu_autotune.hpp:295-333).
  */

@@ -508,17 +508,25 @@ template <typename T> struct TungNl {
 // z-pass kinds.  ZM_PFC: forward both spectra, ETD combine, inverse.
 // ZM_TMF (Tungsten, first z pass): forward Psi, keep the full spectrum, then
 // the inverse of fMF*Psi (the mean field).  ZM_TCOMB (Tungsten, second z
-// pass): forward N, combine with the kept spectrum, inverse.
-enum ZMode { ZM_PFC = 0, ZM_TMF = 1, ZM_TCOMB = 2 };
+// pass): forward N, combine with the kept spectrum, inverse.  ZM_KEEP (PFC
+// runs on the transposed layout that keep Psi's spectrum between steps): the
+// same with the PFC multipliers, the combined spectrum kept in turn.
+enum ZMode { ZM_PFC = 0, ZM_TMF = 1, ZM_TCOMB = 2, ZM_KEEP = 3 };
 
 // Multipliers of one mode for a z pass of kind MODE, scaled by o.scale:
-// (opL, opN) for ZM_PFC, (fMF, -) for ZM_TMF, (expL, nW) for ZM_TCOMB.
+// (opL, opN) for ZM_PFC (ZM_KEEP: opL unscaled, since A carries the scale of the
+// step that kept it), (fMF, -) for ZM_TMF, (expL, nW) for ZM_TCOMB.
 template <int MODE>
 __device__ __forceinline__ void z_mode_ops(const PfcOp &o, const TungOp &p,
                                            double kxy, double kz, double &ma,
                                            double &mb) {
   if constexpr (MODE == ZM_PFC) {
     pfc_op_mode(o, kxy, kz, ma, mb);
+  } else if constexpr (MODE == ZM_KEEP) {
+    PfcOp u = o;
+    u.scale = 1.0;
+    pfc_op_mode(u, kxy, kz, ma, mb);
+    mb *= o.scale;
   } else if constexpr (MODE == ZM_TMF) {
     ma = tung_filter(p, kxy, kz) * o.scale;
     mb = 0.0;

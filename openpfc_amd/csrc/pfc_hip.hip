@@ -710,7 +710,6 @@ int t_pass(pfc_hip_plan_s *p, TStepArgs<T> a, int k, hipStream_t s) {
   const auto &v = t_list<T>(p, t_kind_of_role(role), n)[p->var[role]];
   const cplx<T> *tw = twp<T>(p, v.half ? n / 2 : n, v.plan_id);
   a.tw_x = a.tw_xm = a.tw_y = a.tw_z = tw;
-  if (v.plan_id2 >= 0) a.tw_x = twp<T>(p, 2 * n, v.plan_id2);
   PFC_HIP_TRY(v.fn(a, s), what[k]);
   return 0;
 }
@@ -734,16 +733,48 @@ int step_transposed(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev)
   return 0;
 }
 
-// Whether multi-step PFC runs fuse their step boundaries (role 16).
+// Steps a kept-spectrum run may take before Psi is transformed anew.  The kept
+// half spectrum is not passed through real space, so on its kx = 0 and nx/2
+// planes the part that does not belong to a real field (rounding errors; the C2R
+// drops it) is damped or amplified by opL alone, at most exp(g) per step with g
+// the largest growth exponent L*dt of a mode.  It starts at the rounding level
+// and is harmless while it stays below 1 (its own roundings then stay below the
+// field's): runs of at most 8/g steps keep it under 3000 roundings.  g of the PFC
+// operator: L(k2) = -k2 (eps + (1 - k2)^2) is positive for some k2 < 1 +
+// sqrt(-eps) only.  1 (no kept spectrum) where dt is not positive.
+//
+// Measured, ms per step of a run, tuned variants, kept spectrum against psi
+// transformed anew at a fused boundary (12C) and against single steps (12C + 2R):
+//   FP64 1024^3 18.1 / 21.1 / 23.1 (y 3.14, z 5.35, inverse y 3.47, boundary 4.70)
+//   FP32 1024^3  9.3 / 11.6 / 12.0 (y 1.60, z 2.76, inverse y 1.75, boundary 2.40)
+//   FP64  512^3 2.00 / 2.50 / 2.75,  FP32 512^3 1.07 / 1.34 / 1.42
+//   FP64  256^3 .245 / .334 / .363,  FP32 256^3 .134 / .156 / .188
+int fused_span(const PfcOp &o) {
+  constexpr int kMax = 64;
+  if (!(o.dt > 0)) return 1;
+  if (o.eps >= 0) return kMax;
+  const double top = 1.0 + std::sqrt(-o.eps);
+  double g = 0;
+  for (int i = 1; i <= 512; ++i) {
+    const double k2 = top * i / 512, m = 1.0 - k2;
+    g = std::max(g, -k2 * (o.eps + m * m) * o.dt);
+  }
+  return g * kMax <= 8.0 ? kMax : std::max(1, (int)(8.0 / g));
+}
+
+// Whether multi-step PFC runs keep the spectrum and fuse their step
+// boundaries (role 16).
 template <typename T> bool fused_steps(pfc_hip_plan_s *p) {
   return p->transposed() && !p->tungsten() && p->var[ROLE_STEP_FUSE] == 1 &&
          !t_list<T>(p, TK_X_FUSE, p->role_len(ROLE_T_X_FUSE)).empty();
 }
 
-// nsteps >= 1 PFC steps with fused boundaries: forward x once, then per
-// step the y, z and inverse y passes, with the fused boundary pass between
-// steps, and the inverse x once at the end (4*nsteps + 1 launches).  `ev`
-// (optional) receives 4*nsteps + 2 events around the launches, in order.
+// nsteps >= 1 PFC steps with fused boundaries, in runs of at most fused_span
+// steps: the first step transforms psi and N(psi) (5 passes but the last); the
+// following ones transform N alone (boundary x on T1 of A, forward y A1 -> B2,
+// z with the kept spectrum in A2, inverse y B2 -> A1); the inverse x ends the
+// run.  4*n + 1 launches a run of n.  `ev` (optional) receives 4*nsteps + 2
+// events around the launches of one run of nsteps <= fused_span, in order.
 // (Batched plans: the nsteps steps of field 0, then of field 1, ...; `ev`
 // brackets those of field 0.)
 template <typename T>
@@ -754,16 +785,33 @@ int steps_fused(pfc_hip_plan_s *p, void *psi, int nsteps, hipStream_t s, hipEven
       if (ev && m == 0) (void)hipEventRecord(ev[e++], s);
     };
     const TStepArgs<T> a = pfc_t_args<T>(p, psi, m);
+    const int span = ev ? nsteps : fused_span(a.op);
     mark();
-    for (int i = 0; i < nsteps; ++i) {
-      if (int rc = t_pass<T>(p, a, i == 0 ? 0 : 5, s)) return rc;
-      mark();
-      for (int k = 1; k <= 3; ++k) {
-        if (int rc = t_pass<T>(p, a, k, s)) return rc;
+    for (int done = 0; done < nsteps;) {
+      const int n = std::min(span, nsteps - done);
+      for (int i = 0; i < n; ++i) {
+        TStepArgs<T> f = a; // forward y and z of this step
+        if (i > 0) {
+          f.nfields = 1;
+          f.A2 = a.B2;
+        }
+        TStepArgs<T> z = a;
+        z.mode = i > 0 ? ZM_KEEP : ZM_PFC;
+        z.keep = i + 1 < n;
+        TStepArgs<T> y = a; // inverse y
+        if (i > 0 || z.keep) y.A2 = a.B2;
+        if (int rc = t_pass<T>(p, a, i == 0 ? 0 : 5, s)) return rc;
+        mark();
+        if (int rc = t_pass<T>(p, f, 1, s)) return rc;
+        mark();
+        if (int rc = t_pass<T>(p, z, 2, s)) return rc;
+        mark();
+        if (int rc = t_pass<T>(p, y, 3, s)) return rc;
         mark();
       }
+      if (int rc = t_pass<T>(p, a, 4, s)) return rc;
+      done += n;
     }
-    if (int rc = t_pass<T>(p, a, 4, s)) return rc;
     mark();
   }
   return 0;
@@ -1103,6 +1151,7 @@ template <typename T> void default_variants(pfc_hip_plan_s *p) {
   for (int r = 0; r < ROLE_COUNT; ++r)
     if (plane_role(r) && row_variant_count<T>(p, r) > 0 && plane_variant_default(p))
       p->var[r] = row_variant_count<T>(p, r);
+  p->var[ROLE_STEP_FUSE] = variant_count<T>(p, ROLE_STEP_FUSE) - 1;
 }
 
 int check_plan(pfc_hip_plan_t p) {
@@ -1552,9 +1601,9 @@ int pfc_hip_pfc_step_timed(pfc_hip_plan_t plan, void *psi, int nsteps,
     // launch j of step i is event interval 4*i + j; the exit is 4*nsteps
     for (int k = 0; k < 6; ++k) kernel_ms[k] = 0;
     kernel_ms[0] = span(0);
-    for (int i = 0; i < nsteps; ++i) {
-      if (i > 0) kernel_ms[5] += span((size_t)4 * i) / (nsteps - 1);
-      for (int k = 1; k <= 3; ++k) kernel_ms[k] += span((size_t)4 * i + k) / nsteps;
+    for (int i = 1; i < nsteps; ++i) {
+      kernel_ms[5] += span((size_t)4 * i) / (nsteps - 1);
+      for (int k = 1; k <= 3; ++k) kernel_ms[k] += span((size_t)4 * i + k) / (nsteps - 1);
     }
     kernel_ms[4] = span((size_t)4 * nsteps);
   } else if (!rc) {
@@ -1986,10 +2035,21 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
     return plan->prec == PFC_HIP_F64 ? row_variant_count<double>(plan, role)
                                      : row_variant_count<float>(plan, role);
   };
+  // time of one multi-step call (sets rc)
+  auto run_ms_of = [&](int n) -> double {
+    float ms = 0;
+    hipError_t he = hipEventRecord(ev[0], s);
+    if (he == hipSuccess) rc = pfc_hip_pfc_step(plan, psi, n, s);
+    if (rc) return 1e300;
+    if (he == hipSuccess) he = hipEventRecord(ev[1], s);
+    if (he == hipSuccess) he = hipEventSynchronize(ev[1]);
+    if (he == hipSuccess) he = hipEventElapsedTime(&ms, ev[0], ev[1]);
+    if (he != hipSuccess)
+      rc = fail(PFC_HIP_EDEVICE, std::string("autotune run: ") + hipGetErrorString(he));
+    return rc ? 1e300 : (double)ms;
+  };
   int slot = 0;
   double layout_ms[2] = {0, 0};
-  double role_best[ROLE_COUNT];
-  for (double &b : role_best) b = 1e300;
   // both layouts when the plan has both (natural first, slot order); a
   // double-butterfly plan has the transposed one only
   const bool two = plan->t_ok && !plan->xp;
@@ -2047,7 +2107,6 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
         }
       }
       plan->var[sp.role] = best_v;
-      role_best[sp.role] = best;
       slot += count + (plane_slot[sp.role] >= 0 ? 1 : 0);
     }
     // The plane kernels against the tuned row and column kernels, by the time
@@ -2072,18 +2131,8 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
         apply(m);
         double t = 1e300;
         for (int r = 0; r <= reps && !rc; ++r) {
-          float ms = 0;
-          hipError_t he = hipEventRecord(ev[0], s);
-          if (he == hipSuccess) rc = pfc_hip_pfc_step(plan, psi, kRun, s);
-          if (rc) break;
-          if (he == hipSuccess) he = hipEventRecord(ev[1], s);
-          if (he == hipSuccess) he = hipEventSynchronize(ev[1]);
-          if (he == hipSuccess) he = hipEventElapsedTime(&ms, ev[0], ev[1]);
-          if (he != hipSuccess) {
-            rc = fail(PFC_HIP_EDEVICE, std::string("autotune run: ") + hipGetErrorString(he));
-            break;
-          }
-          if (r > 0) t = std::min(t, (double)ms / kRun);
+          const double ms = run_ms_of(kRun);
+          if (r > 0) t = std::min(t, ms / kRun);
         }
         for (size_t i = 0; i < pr.size(); ++i) // reported: the fastest step with the role on
           if ((m >> i & 1) && times_ms && plane_slot[pr[i]] < max_times) {
@@ -2137,12 +2186,16 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
       }
       plan->var[ROLE_T_X_FUSE] = best_v;
       slot += count;
-      // fuse step boundaries when one fused pass beats the two it replaces
-      // by a clear margin (the two timings come from different launches)
-      constexpr double kFuseMargin = 0.95;
-      if (count > 0)
-        plan->var[ROLE_STEP_FUSE] =
-            best < kFuseMargin * (role_best[ROLE_T_X_FWD] + role_best[ROLE_T_X_INV]) ? 1 : 0;
+      // kept-spectrum runs against single steps, by the time of whole runs
+      double run_ms[2] = {1e300, 1e300};
+      for (int fuse = 0; fuse < 2 && count > 0 && !rc; ++fuse) {
+        plan->var[ROLE_STEP_FUSE] = fuse;
+        for (int r = 0; r <= reps && !rc; ++r) {
+          const double ms = run_ms_of(6);
+          if (r > 0) run_ms[fuse] = std::min(run_ms[fuse], ms);
+        }
+      }
+      if (count > 0) plan->var[ROLE_STEP_FUSE] = run_ms[1] < run_ms[0] ? 1 : 0;
     }
     double fastest = 1e300, pm[9];
     for (int r = 0; r <= reps && !rc; ++r) {

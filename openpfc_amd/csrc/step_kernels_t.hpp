@@ -89,6 +89,7 @@ __device__ __forceinline__ void fetch_partner(const cplx<T> (&v)[E], cplx<T> (&p
 template <typename T> struct TStepArgs {
   Nonlin<T> nl;     // nonlinearity (plain or mean-split)
   int zero_k0;      // mean-split step: keep the k = 0 mode of the deviation at 0
+  int keep;         // z pass: store the combined spectrum in A2, its inverse in B2
   int mode;         // k_tz kind (ZMode)
   int nfields;      // k_ty_fwd: 2 (A and B) or 1 (A only)
   TungOp top;       // Tungsten operator scalars
@@ -329,6 +330,20 @@ __device__ __forceinline__ void tile_store(const T *sr, const T *si, int nvalid,
   }
 }
 
+// ZM_PFC with a.keep set and ZM_KEEP are the z passes of a kept-spectrum run: the
+// combined spectrum stays in A (the next step's Psi, forward transforms
+// included) and its inverse goes to B.  ZM_KEEP takes A as such a spectrum, so
+// only N is transformed forward.
+// opL*h + opN*v of one mode; double-butterfly plans combine unrounded in double.
+template <typename Plan, typename T, typename M>
+__device__ __forceinline__ cplx<T> z_combine(cplx<T> h, cplx<T> v, M opl, M opn) {
+  if constexpr (Plan::XP)
+    return cplx<T>{(T)((double)h.x * opl + (double)v.x * opn),
+                   (T)((double)h.y * opl + (double)v.y * opn)};
+  else
+    return c_add(c_scale(h, (T)opl), c_scale(v, (T)opn));
+}
+
 template <typename T, typename Plan, int G, bool SPLIT, int MODE, bool PRE = false,
           bool NT = false>
 __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
@@ -420,13 +435,19 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const cplx<T> h = PRE ? acc[e] : ld_line<NT>(la + (t + TL * e));
-        acc[e] = c_add(c_scale(h, (T)opl[e]), c_scale(v[e], (T)opn[e]));
+        acc[e] = z_combine<Plan>(h, v[e], opl[e], opn[e]);
       }
+      if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
     }
+  }
+  if ((MODE == ZM_PFC || MODE == ZM_KEEP) && a.keep && active) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) st_line<NT>(la + (t + TL * e), acc[e]);
   }
   LineFft<T, Plan, +1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
   if (active) {
-    cplx<T> *__restrict__ out = MODE == ZM_TMF ? lb : la;
+    cplx<T> *__restrict__ out =
+        (MODE == ZM_TMF || MODE == ZM_KEEP || (MODE == ZM_PFC && a.keep)) ? lb : la;
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<NT>(out + (t + TL * e), acc[e]);
   }
@@ -536,15 +557,21 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz_mt(TStepArgs<T> a) {
     }
     if (a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
   } else {
-    // A = Fz^-1(expL*A + nW*Fz(B)), A already a full spectrum
+    // ma*A + mb*Fz(B), A already a full spectrum
     LineFft<T, Plan, -1, SPLIT, true, row_wave<Plan>()>::run(v, t, ll, a.tw_z);
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      acc[e] = c_add(c_scale(acc[e], (T)ta[slot(e)]), c_scale(v[e], (T)tb[slot(e)]));
+      acc[e] = z_combine<Plan>(acc[e], v[e], ta[slot(e)], tb[slot(e)]);
+    if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
+  }
+  if ((MODE == ZM_PFC || MODE == ZM_KEEP) && a.keep && active) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) st_line<true>(la + (t + TL * e), acc[e]);
   }
   LineFft<T, Plan, +1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
   if (active) {
-    cplx<T> *__restrict__ out = MODE == ZM_TMF ? lb : la;
+    cplx<T> *__restrict__ out =
+        (MODE == ZM_TMF || MODE == ZM_KEEP || (MODE == ZM_PFC && a.keep)) ? lb : la;
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<true>(out + (t + TL * e), acc[e]);
   }
@@ -1074,77 +1101,63 @@ __global__ void __launch_bounds__(G *Plan::TL) k_ty_inv_w(TStepArgs<T> a) {
 
 
 // ----------------------------------------------------------------------------
-// Step boundary of a multi-step PFC run, fused: the inverse x pass of step n
-// (T1 rows of Psi -> psi, nx/2-point plan PH) and the forward x pass of step
-// n+1 (psi -> A1: Psi, B1: N, nx-point plan PF) for G consecutive rows of
-// plane z, psi never leaving the block.  The C2R leaves psi as the pairs
-// (psi[2m], psi[2m+1]) of m = t + TL*e; one LDS exchange hands each thread
-// the positions t + TL*e of the nx-point ownership, then the forward x runs
-// as in k_tx_fwd_w.  PH and PF use the same threads per line.  Reads C and
-// writes 2C: 2R less than the two passes it replaces.  A block reads and then
-// rewrites only its own (z, y-group) tile of A1.
+// Step boundary of a kept-spectrum PFC run, on T1 in place: for G consecutive
+// rows of plane z the half spectra of Psi are loaded transposed and brought to
+// real space (nx/2-point C2R), the nonlinearity is formed in registers and
+// transformed forward (nx/2-point R2C of the same pairs, so no exchange moves
+// psi), and its half spectra go back to the tile they came from.  Psi's own
+// spectrum is kept by the z pass, so the boundary reads C and writes C; it
+// used to write Psi's half spectra too (C + 2C, through one nx-point
+// transform): 6.40 ms at 1024^3 FP64, 3.42 ms in FP32, against the figures at
+// fused_span (pfc_hip.hip).
+//
+// What bounds it: memory latency at two blocks per CU (the staging tile is 66 KB
+// for 8 rows of 1024 doubles).  WPE > 1 caps the registers so that WPE waves
+// fit on a SIMD.
 // ----------------------------------------------------------------------------
-template <typename T, typename PH, typename PF, int G, bool SPLIT> constexpr int tx_fuse_lds() {
-  constexpr int inv = tx_inv_lds<T, PH, G, true>();
-  constexpr int xch = G * row_padded(PF::N);
-  constexpr int fwd = tx_fwd_w_lds<T, PF, G, SPLIT>();
-  return inv > xch ? (inv > fwd ? inv : fwd) : (xch > fwd ? xch : fwd);
-}
-
-// WPE > 1 caps the registers so that WPE waves fit on a SIMD.
-template <typename T, typename PH, typename PF, int G, bool SPLIT, int WPE = 1>
-__global__ void __launch_bounds__(G *PF::TL, WPE) k_tx_fuse(TStepArgs<T> a) {
-  static_assert(PH::TL == PF::TL && PF::N == 2 * PH::N, "paired plans");
-  constexpr int TL = PH::TL, EH = PH::E, EF = PF::E, M = PH::N;
-  constexpr int RPH = row_padded(M), RPF = row_padded(PF::N);
-  constexpr int PLH = t_plane<PH, G>();
-  constexpr int W = M + 1;
-  __shared__ T lds[tx_fuse_lds<T, PH, PF, G, SPLIT>()];
+template <typename T, typename Plan, int G, int WPE = 1, bool NT = false>
+__global__ void __launch_bounds__(G *Plan::TL, WPE) k_tx_bnd(TStepArgs<T> a) {
+  constexpr int TL = Plan::TL, E = Plan::E, M = Plan::N, RP = row_padded(M);
+  constexpr int PL = t_plane<Plan, G>(), W = M + 1;
+  __shared__ T lds[tx_inv_lds<T, Plan, G, true>()];
   const int t = threadIdx.x % TL, g = threadIdx.x / TL;
   const int ngy = (a.ny + G - 1) / G;
   const unsigned bid = xcd_block<T, G>(blockIdx.x, gridDim.x);
   const int z = (int)bid / ngy, y0 = ((int)bid % ngy) * G;
+  cplx<T> *__restrict__ spec = a.A1 + (long)z * a.W * a.ny + y0;
+  T *sr = lds, *si = lds + W * tile_pitch<G, T>();
 
-  // inverse x: transposed load of the G rows, C2R merge, inverse transform
-  cplx<T> v[EH];
-  {
-    T *sr = lds, *si = lds + W * tile_pitch<G, T>();
-    const cplx<T> *__restrict__ src = a.A1 + (long)z * a.W * a.ny + y0;
-    tile_load<W, G, G * TL, false>(sr, si, a.ny - y0,
-                                   [&](int kx, int gg) { return src + ((long)kx * a.ny + gg); });
-    __syncthreads();
-#pragma unroll
-    for (int e = 0; e < EH; ++e) {
-      const int k = t + TL * e;
-      v[e] = c2r_merge(cplx<T>{sr[tile_idx<G, T>(k, g)], si[tile_idx<G, T>(k, g)]},
-                       cplx<T>{sr[tile_idx<G, T>(M - k, g)], si[tile_idx<G, T>(M - k, g)]},
-                       a.wn[k], k == 0);
-    }
-    __syncthreads(); // the staging area becomes the FFT exchange area
-  }
-  const LdsLine<T> llh{lds, g * RPH, 1, PLH};
-  LineFft<T, PH, +1, false, true, row_wave<PH>()>::run(v, t, llh, a.tw_xm);
-
-  // psi to the nx-point ownership, then psi + i*N(psi)
+  tile_load<W, G, G * TL, NT>(sr, si, a.ny - y0,
+                              [&](int kx, int gg) { return spec + ((long)kx * a.ny + gg); });
   __syncthreads();
-  T *row = lds + g * RPF;
+  cplx<T> v[E];
 #pragma unroll
-  for (int e = 0; e < EH; ++e) {
-    // positions 2m and 2m + 1 of m = t + TL*e: pad_pos(2m) = row_slot<2TL>(2t, e)
-    // (2m mod 16 <= 14, so 2m + 1 lands in the next slot)
-    const int i = row_slot<2 * TL>(2 * t, e);
-    row[i] = v[e].x;
-    row[i + 1] = v[e].y;
+  for (int e = 0; e < E; ++e) {
+    const int k = t + TL * e;
+    v[e] = c2r_merge(cplx<T>{sr[tile_idx<G, T>(k, g)], si[tile_idx<G, T>(k, g)]},
+                     cplx<T>{sr[tile_idx<G, T>(M - k, g)], si[tile_idx<G, T>(M - k, g)]},
+                     a.wn[k], k == 0);
+  }
+  __syncthreads(); // the staging area becomes the FFT exchange area
+  const LdsLine<T> ll{lds, g * RP, 1, PL};
+  LineFft<T, Plan, +1, false, true, row_wave<Plan>()>::run(v, t, ll, a.tw_xm);
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = cplx<T>{a.nl(v[e].x), a.nl(v[e].y)};
+  cplx<T> xm;
+  row_r2c<T, Plan, G>(v, xm, lds, t, g, a.tw_xm, a.wn);
+  __syncthreads(); // every row is done with the exchange area
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    sr[tile_idx<G, T>(t + TL * e, g)] = v[e].x;
+    si[tile_idx<G, T>(t + TL * e, g)] = v[e].y;
+  }
+  if (t == 0) {
+    sr[tile_idx<G, T>(M, g)] = xm.x;
+    si[tile_idx<G, T>(M, g)] = xm.y;
   }
   __syncthreads();
-  cplx<T> w[EF];
-#pragma unroll
-  for (int e = 0; e < EF; ++e) {
-    const T u = row[row_slot<TL>(t, e)];
-    w[e] = cplx<T>{u, a.nl(u)};
-  }
-  __syncthreads(); // the LDS becomes the forward transform's exchange area
-  fwd_split_store_wide<T, PF, G, SPLIT>(w, lds, t, g, z, y0, a);
+  tile_store<W, G, G * TL, NT>(sr, si, a.ny - y0,
+                               [&](int kx, int gg) { return spec + ((long)kx * a.ny + gg); });
 }
 
 } // namespace pfc_amd

@@ -71,6 +71,9 @@ pfc_hip_plan_t plan_for(int nx, int ny, int nz, int prec) {
   if (!p) {
     p = std::make_unique<Plan>();
     check(pfc_hip_plan_create(nx, ny, nz, prec, 0, &p->h), "pfc_trajectory: plan");
+    // a state recomputed from a checkpoint has to be the state of the forward
+    // run bit for bit, however many steps a call takes
+    check(pfc_hip_variant_set(p->h, PFC_HIP_ROLE_STEP_FUSE, 0), "pfc_trajectory: single steps");
   }
   return p->h;
 }

@@ -31,8 +31,8 @@ enum Role {
   ROLE_X_TUNG = 12,     // Tungsten natural step: fused inverse x, N, forward x
   ROLE_T_X_R2C = 13,    // Tungsten transposed step: psi -> T1 (psi only)
   ROLE_T_X_TUNG = 14,   // Tungsten transposed step: fused x pass on T1
-  ROLE_T_X_FUSE = 15,   // PFC multi-step run: inverse x of one step fused with the next forward x
-  ROLE_STEP_FUSE = 16,  // 0: multi-step runs as single steps, 1: fused step boundaries
+  ROLE_T_X_FUSE = 15,   // PFC multi-step run: step boundary (inverse x, N, forward x of N)
+  ROLE_STEP_FUSE = 16,  // 0: multi-step runs as single steps, 1: kept spectrum, fused boundaries
   ROLE_COUNT = 17
 };
 
@@ -75,7 +75,6 @@ template <typename T> struct TV {
   int plan_id;
   hipError_t (*fn)(TStepArgs<T> a, hipStream_t s);
   int half = 0; // 1: the kernel runs the n/2-point plan `plan_id` of a length-n role
-  int plan_id2 = -1; // >= 0: also the 2n-point plan plan_id2 (its twiddles in tw_x)
 };
 
 // Variant lists for a line length n (empty when n is unsupported).

@@ -356,6 +356,9 @@ hipError_t tz_launch(TStepArgs<T> a, hipStream_t s) {
   case ZM_TCOMB:
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB>), grid, block, 0, s, a);
     break;
+  case ZM_KEEP:
+    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP>), grid, block, 0, s, a);
+    break;
   default:
     return hipErrorInvalidValue;
   }
@@ -421,25 +424,8 @@ hipError_t tz_pre_launch(TStepArgs<T> a, hipStream_t s) {
   case ZM_TCOMB:
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB, true>), grid, block, 0, s, a);
     break;
-  default:
-    return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-// z pass with non-temporal line loads and stores (k_tz<..., NT = true>)
-template <typename T, typename Plan, int G, bool S, bool PRE>
-hipError_t tz_nt_launch(TStepArgs<T> a, hipStream_t s) {
-  const long lines = (long)a.W * a.ny;
-  dim3 grid((unsigned)((lines + G - 1) / G)), block(G * Plan::TL);
-  switch (a.mode) {
-  case ZM_PFC:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_PFC, PRE, true>), grid, block, 0, s, a);
-    break;
-  case ZM_TMF:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TMF, PRE, true>), grid, block, 0, s, a);
-    break;
-  case ZM_TCOMB:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB, PRE, true>), grid, block, 0, s, a);
+  case ZM_KEEP:
+    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP, true>), grid, block, 0, s, a);
     break;
   default:
     return hipErrorInvalidValue;
@@ -462,6 +448,9 @@ hipError_t tz_mt_launch(TStepArgs<T> a, hipStream_t s) {
     break;
   case ZM_TCOMB:
     hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_TCOMB, PAIR>), grid, block, 0, s, a);
+    break;
+  case ZM_KEEP:
+    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_KEEP, PAIR>), grid, block, 0, s, a);
     break;
   default:
     return hipErrorInvalidValue;
@@ -487,10 +476,10 @@ hipError_t tx_tung_wide_o_launch(TStepArgs<T> a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <typename T, typename PH, typename PF, int G, bool S, int WPE = 1>
-hipError_t tx_fuse_launch(TStepArgs<T> a, hipStream_t s) {
-  dim3 grid((unsigned)(a.nz * ((a.ny + G - 1) / G))), block(G * PF::TL);
-  hipLaunchKernelGGL((k_tx_fuse<T, PH, PF, G, S, WPE>), grid, block, 0, s, a);
+template <typename T, typename Plan, int G, int WPE, bool NT>
+hipError_t tx_bnd_launch(TStepArgs<T> a, hipStream_t s) {
+  dim3 grid((unsigned)(a.nz * ((a.ny + G - 1) / G))), block(G * Plan::TL);
+  hipLaunchKernelGGL((k_tx_bnd<T, Plan, G, WPE, NT>), grid, block, 0, s, a);
   return hipGetLastError();
 }
 
@@ -620,13 +609,6 @@ void add_t_z_pre(std::vector<TV<T>> &v, int pid) {
                      "/pre",
                  pid, &tz_pre_launch<T, Plan, G, S>});
 }
-template <typename T, typename Plan, int G, bool S, bool PRE>
-void add_t_z_nt(std::vector<TV<T>> &v, int pid) {
-  if constexpr (t_fits<T, Plan, G, S, true, TK_Z>())
-    v.push_back({plan_name<Plan>() + "/G" + std::to_string(G) + (S ? "/split" : "/full") +
-                     (PRE ? "/pre" : "") + "/nt",
-                 pid, &tz_nt_launch<T, Plan, G, S, PRE>});
-}
 template <typename T, typename Plan, int G, bool S, bool PAIR = false>
 void add_t_z_mt(std::vector<TV<T>> &v, int pid) {
   if constexpr (t_fits<T, Plan, G, S, true, TK_Z>() && (!PAIR || G == 2) &&
@@ -637,19 +619,15 @@ void add_t_z_mt(std::vector<TV<T>> &v, int pid) {
                      (PAIR ? "/mtp" : "/mt"),
                  pid, &tz_mt_launch<T, Plan, G, S, PAIR>});
 }
-// Fused step boundary (k_tx_fuse): an nx/2-point plan PH paired with an
-// nx-point plan PF of the same threads per line; WPE > 1 caps the registers
-// for WPE waves per SIMD (named /wN).
-template <typename T, typename PH, typename PF, int G, bool S, int WPE = 1>
-void add_t_fuse(std::vector<TV<T>> &v, int pid, int pid2) {
-  if constexpr (PH::TL == PF::TL && G * PF::TL <= kMaxThreads && G * PF::TL >= 64 &&
-                tx_fuse_lds<T, PH, PF, G, S>() * (int)sizeof(T) <= kMaxLds) {
-    TV<T> e{plan_name<PH>() + "+" + plan_name<PF>() + "/G" + std::to_string(G) +
-                (S ? "/split" : "/full") + (WPE > 1 ? "/w" + std::to_string(WPE) : ""),
-            pid, &tx_fuse_launch<T, PH, PF, G, S, WPE>};
-    e.plan_id2 = pid2;
-    v.push_back(e);
-  }
+// Step boundary of kept-spectrum runs (k_tx_bnd); WPE > 1 caps the registers for
+// WPE waves per SIMD (named /wN).
+template <typename T, typename Plan, int G, int WPE = 1, bool NT = false>
+void add_t_bnd(std::vector<TV<T>> &v, int pid) {
+  if constexpr (G * Plan::TL <= kMaxThreads && G * Plan::TL >= 64 &&
+                tx_inv_lds<T, Plan, G, true>() * (int)sizeof(T) <= kMaxLds)
+    v.push_back({plan_name<Plan>() + "/G" + std::to_string(G) +
+                     (WPE > 1 ? "/w" + std::to_string(WPE) : "") + (NT ? "/nt" : ""),
+                 pid, &tx_bnd_launch<T, Plan, G, WPE, NT>});
 }
 // Tungsten fused x pass, wide store, registers capped for WPE waves per SIMD
 template <typename T, typename Plan, int G, int WPE>
@@ -732,10 +710,6 @@ template <typename T, int N, int KIND> std::vector<TV<T>> make_t_kind() {
         add_t_z_pre<T, P, 1, true>(v, pid);
         add_t_z_pre<T, P, 1, false>(v, pid);
         add_t_z_pre<T, P, 2, true>(v, pid);
-        add_t_z_nt<T, P, 1, true, false>(v, pid);
-        add_t_z_nt<T, P, 1, false, false>(v, pid);
-        add_t_z_nt<T, P, 1, true, true>(v, pid);
-        add_t_z_nt<T, P, 1, false, true>(v, pid);
         // tabulated multipliers: one wavefront of lines per block at least
         constexpr int GM = P::TL >= 64 ? 1 : 64 / P::TL;
         add_t_z_mt<T, P, GM, true>(v, pid);
@@ -746,30 +720,20 @@ template <typename T, int N, int KIND> std::vector<TV<T>> make_t_kind() {
       });
     }
     if constexpr (KIND == TK_X_FUSE) {
-      // N is nx/2 here; the forward half of the pass runs the 2N-point plans
-      if constexpr (2 * N <= 1024) {
-        for_t_plans<T, N>(typename Plans<N>::L{}, [&](auto ph, int pid) {
-          using PH = decltype(ph);
-          for_t_plans<T, 2 * N>(typename Plans<2 * N>::L{}, [&](auto pf, int pid2) {
-            using PF = decltype(pf);
-            constexpr int G0 = 128 / (2 * (int)sizeof(T));
-            add_t_fuse<T, PH, PF, G0 / 2, true>(v, pid, pid2);
-            add_t_fuse<T, PH, PF, G0 / 2, false>(v, pid, pid2);
-            add_t_fuse<T, PH, PF, G0, true>(v, pid, pid2);
-            add_t_fuse<T, PH, PF, G0, false>(v, pid, pid2);
-            // registers capped so that the blocks the LDS allows all fit: four of
-            // G0 / 2 lines or two of G0 lines (128-byte stores) per CU
-            if constexpr (4 * tx_fuse_lds<T, PH, PF, G0 / 2, true>() * (int)sizeof(T) <=
-                              160 * 1024 &&
-                          (G0 / 2) * PF::TL / 64 <= 8)
-              add_t_fuse<T, PH, PF, G0 / 2, true, 4 * (G0 / 2) * PF::TL / 256>(v, pid, pid2);
-            if constexpr (2 * tx_fuse_lds<T, PH, PF, G0, true>() * (int)sizeof(T) <=
-                              160 * 1024 &&
-                          G0 * PF::TL / 128 <= 8 && G0 * PF::TL / 128 > 1)
-              add_t_fuse<T, PH, PF, G0, true, 2 * G0 * PF::TL / 256>(v, pid, pid2);
-          });
-        });
-      }
+      for_t_plans<T, N>(typename Plans<N>::L{}, [&](auto p, int pid) {
+        using P = decltype(p);
+        constexpr int G0 = 128 / (2 * (int)sizeof(T));
+        add_t_bnd<T, P, G0>(v, pid);
+        add_t_bnd<T, P, G0 / 2>(v, pid);
+        add_t_bnd<T, P, G0, 1, true>(v, pid);
+        // registers capped so that the blocks the LDS allows all fit
+        constexpr int lds = tx_inv_lds<T, P, G0, true>() * (int)sizeof(T);
+        constexpr int blocks = 160 * 1024 / lds, wpe = blocks * (G0 * P::TL / 64) / 4;
+        if constexpr (wpe > 1 && wpe <= 8) {
+          add_t_bnd<T, P, G0, wpe>(v, pid);
+          add_t_bnd<T, P, G0, wpe, true>(v, pid);
+        }
+      });
     }
     if constexpr (KIND == TK_X_R2C || KIND == TK_X_TUNG) {
       for_t_plans<T, N>(typename Plans<N>::L{}, [&](auto p, int pid) {
@@ -826,8 +790,6 @@ template <int N, int KIND> std::vector<TV<float>> make_t_kind_xp() {
       add_t<T, P, G, true, true, KIND>(v, id);
       add_t<T, P, G, false, true, KIND>(v, id);
       add_t_z_pre<T, P, G, false>(v, id);
-      add_t_z_nt<T, P, G, false, true>(v, id);
-      add_t_z_nt<T, P, G, true, false>(v, id);
       add_t<T, P, 2 * G, true, true, KIND>(v, id);
       add_t_z_mt<T, P, G, false>(v, id);
       add_t_z_mt<T, P, G, true>(v, id);
