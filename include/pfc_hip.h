@@ -396,8 +396,8 @@ int pfc_hip_tungsten_operators(pfc_hip_plan_t plan, void *filterMF, void *expL,
  * z plane of the half spectrum fits a CU's LDS: a block then does the x and the
  * y pass of a whole plane (role 2 is not used in that direction), and where both
  * directions of the PFC step are on it a multi-step run makes each step boundary
- * in one launch, with the bits of single steps.  A new plan starts on "plane"
- * where that is measured faster, and on index 0 of the other roles but 16.  No reference
+ * in one launch, with the bits of single steps.  A new plan starts on the
+ * variants measured fastest for its line lengths and precision.  No reference
  * counterpart: the reference delegates shapes to rocFFT; its GPU autotuner only
  * times 1-D block sizes (include/openpfc/runtime/common/gpu_autotune.hpp:295-333).
  */
@@ -440,7 +440,8 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index);
  * (Tungsten); roles of an unsupported layout contribute no entries (role 15,
  * the fused step boundary, is timed on its own launches).  Then
  * follow the fastest step times of the transposed and of the natural layout (0 if
- * not run); up to max_times entries are written.
+ * not run; PFC: single steps or steps of a run, whichever is faster); up to
+ * max_times entries are written.
  */
 int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
                          double *times_ms, int max_times);

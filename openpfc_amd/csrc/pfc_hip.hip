@@ -13,6 +13,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <new>
 #include <string>
 #include <map>
@@ -139,6 +140,7 @@ struct pfc_hip_plan_s {
   bool mean_split = false; // field holds psi - mean; mean kept in double here
   double mean = 0.0;
   int var[ROLE_COUNT] = {};
+  bool z_default = true; // the transposed z variant is still the default's
   size_t bytes = 0;
   // Batched plans step `batch` fields of these extents stored one after
   // another.  The natural layout steps them all in each launch, reading
@@ -1146,8 +1148,159 @@ bool plane_variant_default(const pfc_hip_plan_s *p) {
   return b > 0 && b <= 140 * 1024 && (p->nz >= 64 || b <= (size_t)1600 * p->nz);
 }
 
+// Default variants by line length, where another variant than the first of a
+// role's list measured faster over the grids of that length (role sweeps on
+// 256x128x128 to 1024^3 for the transposed roles, 16x1024x64 to 1024^3 for the
+// natural ones, both models; the ratio to each sweep's best was 1.00 to 1.05 for
+// these and is given below for the first of the list).  What they have in
+// common: 128 contiguous bytes per strided access (8 lines of doubles, 16 of
+// floats), few wide transposition rounds instead of one per value, non-temporal
+// lines, a z table per line; 8 values a thread in double up to 512 points, where
+// 16 leave one or two waves per SIMD.  Single precision takes no plan with more
+// radix passes (roundings) than the first of its list.
+struct DefaultVariant {
+  int role, n;
+  const char *name;
+};
+constexpr DefaultVariant kDefaultF64[] = {
+    // natural layout
+    {ROLE_PFC_Z, 96, "r4x4x6/E12/L8/full"},            // first 1.24
+    {ROLE_PFC_Z, 128, "r8x4x4/E8/L8/full"},            // 1.09 to 1.17
+    {ROLE_PFC_Z, 256, "r8x8x4/E8/L8/full"},            // 1.22 at 512x32x256
+    {ROLE_PFC_Z, 512, "r8x8x8/E8/L4/full"},            // 1.08
+    {ROLE_COL_Y, 96, "r4x4x6/E12/L8/full"},            // 1.09
+    {ROLE_COL_Y, 512, "r8x8x8/E8/L8/full"},            // 1.05 to 1.09
+    {ROLE_COL_Z, 96, "r4x4x6/E12/L8/full"},            // as the y columns
+    {ROLE_COL_Z, 512, "r8x8x8/E8/L8/full"},
+    {ROLE_PFC_X, 256, "r8x8x4/E8/rows8"},              // 1.03 to 1.06
+    {ROLE_X_R2C, 128, "r8x4x4/E8/rows8"},              // 1.14, 1.21
+    {ROLE_X_R2C, 256, "r4x4x4x4/E4/rows1"},            // 1.08
+    {ROLE_X_C2R, 128, "r8x4x4/E8/rows16"},             // 1.07 to 1.12
+    {ROLE_X_C2R, 256, "r4x4x4x4/E4/rows2"},            // 1.02 to 1.11
+    {ROLE_X_C2R, 512, "r16x16x2/E16/rows4"},           // 1.13
+    {ROLE_X_TUNG, 128, "r8x4x4/E8/rows4"},             // 1.24, 1.52
+    {ROLE_X_TUNG, 256, "r4x4x4x4/E4/rows1"},           // 1.05
+    // transposed layout
+    {ROLE_T_X_FWD, 256, "r4x4x4x4/E4/G8/split/wide/nt"},    // 1.00 to 1.16
+    {ROLE_T_X_FWD, 512, "r8x8x8/E8/G8/full/wide/nt"},       // 1.15
+    {ROLE_T_X_FWD, 1024, "r16x16x4/E16/G8/split/wide/nt"},  // 1.02, 1.04
+    {ROLE_T_Y_FWD, 128, "r8x4x4/E8/G8/split/wide4/nt"},     // 1.06, 1.11
+    {ROLE_T_Y_FWD, 256, "r16x16/E16/G8/split/wide4/nt"},    // 1.02 to 1.28
+    {ROLE_T_Y_FWD, 512, "r8x8x8/E8/G8/split/wide1/nt"},     // 1.13, 1.16
+    {ROLE_T_Y_FWD, 1024, "r16x16x4/E16/G8/split/wide2/nt"}, // 1.08
+    {ROLE_T_Z, 128, "r8x4x4/E8/G4/split/mt"},               // 1.29 to 1.44
+    {ROLE_T_Z, 256, "r8x8x4/E8/G2/split/pre"},              // 1.13 to 1.26
+    {ROLE_T_Z, 512, "r8x8x8/E8/G1/full/mt"},                // 1.25
+    {ROLE_T_Z, 1024, "r16x16x4/E16/G1/split/mt"},           // 1.16
+    {ROLE_T_Y_INV, 128, "r8x4x4/E8/G8/split/wide4/nt"},     // 1.37
+    {ROLE_T_Y_INV, 256, "r16x16/E16/G8/split/wide2"},       // 1.03 to 1.22
+    {ROLE_T_Y_INV, 512, "r16x16x2/E16/G8/split/wide2"},     // 1.04, 1.06
+    {ROLE_T_Y_INV, 1024, "r16x16x4/E16/G8/split/wide2"},    // 1.01, 1.20
+    {ROLE_T_X_INV, 128, "r8x4x4/E8/G8/nt"},                 // 1.01 to 1.25
+    {ROLE_T_X_INV, 256, "r8x8x4/E8/G8/nt"},                 // 1.04 to 1.19
+    {ROLE_T_X_INV, 512, "r16x16x2/E16/G8/nt"},              // 1.03, 1.07
+    {ROLE_T_X_FUSE, 128, "r8x4x4/E8/G8/w4"},                // 1.00 to 1.09
+    {ROLE_T_X_FUSE, 256, "r8x8x4/E8/G8/w4"},                // 1.07, 1.09
+    {ROLE_T_X_FUSE, 512, "r16x16x2/E16/G8/w2"},             // 1.04, 1.06
+    {ROLE_T_X_R2C, 128, "r8x4x4/E8/G8"},                    // 1.06, 1.10
+    {ROLE_T_X_TUNG, 128, "r8x4x4/E8/G8/wide"},              // 1.05, 1.15
+    {ROLE_T_X_TUNG, 256, "r8x8x4/E8/G8/wide/w4"},           // 1.04
+    {ROLE_T_X_TUNG, 512, "r8x8x8/E8/G8/wide/w4"}};          // 1.25 (1024^3)
+constexpr DefaultVariant kDefaultF32[] = {
+    {ROLE_PFC_Z, 512, "r8x8x8/E8/L8/full"},                  // first 1.13
+    {ROLE_PFC_Z, 1024, "r16x16x4/E16/L8/full"},              // 1.77, 2.40
+    {ROLE_COL_Y, 512, "r8x8x8/E8/L16/full"},                 // 1.02
+    {ROLE_COL_Y, 1024, "r16x16x4/E16/L8/full"},              // 1.06
+    {ROLE_COL_Z, 512, "r8x8x8/E8/L16/full"},                 // as the y columns
+    {ROLE_COL_Z, 1024, "r16x16x4/E16/L8/full"},
+    {ROLE_PFC_X, 256, "r16x16/E16/rows8"},                   // 1.01, 1.11
+    {ROLE_T_X_FWD, 256, "r16x16/E16/G16/full/wide/nt"},      // 1.10, 1.27
+    {ROLE_T_X_FWD, 512, "r8x8x8/E8/G16/split/wide/nt"},      // 1.07, 1.33
+    {ROLE_T_X_FWD, 1024, "r16x16x4/E16/G16/split/wide/nt"},  // 1.11, 1.17
+    {ROLE_T_Y_FWD, 256, "r16x16/E16/G16/split/wide2"},       // 1.02 to 1.04
+    {ROLE_T_Y_FWD, 512, "r8x8x8/E8/G16/split/wide1/nt"},     // 1.02, 1.05
+    {ROLE_T_Y_FWD, 1024, "r16x16x4/E16/G16/split/wide2/nt"}, // 1.20
+    {ROLE_T_Z, 128, "r16x8/E16/G8/full/mt"},                 // 1.04 to 1.52
+    {ROLE_T_Z, 256, "r16x16/E16/G4/split/mt"},               // 1.29 to 1.36
+    {ROLE_T_Z, 512, "r8x8x8/E8/G2/split/mtp"},               // 1.37
+    {ROLE_T_Z, 1024, "r16x16x4/E16/G2/split/mtp"},           // 1.73
+    {ROLE_T_Y_INV, 128, "r16x8/E16/G16/split/wide2/nt"},     // 1.76, 1.79
+    {ROLE_T_Y_INV, 256, "r16x16/E16/G16/split/wide2"},       // 1.24 to 1.34
+    {ROLE_T_Y_INV, 512, "r16x16x2/E16/G16/split/wide2"},     // 1.16, 1.21
+    {ROLE_T_Y_INV, 1024, "r16x16x4/E16/G16/split/wide2"},    // 1.08
+    {ROLE_T_X_INV, 512, "r8x8x8/E8/G16/nt"},                 // 1.05, 1.35
+    {ROLE_T_X_FUSE, 128, "r16x8/E16/G8"},                    // 1.04, 1.06
+    {ROLE_T_X_FUSE, 512, "r16x16x2/E16/G16/nt"},             // 1.19, 1.29
+    {ROLE_T_X_TUNG, 256, "r16x16/E16/G16/wide"}};            // 1.01
+// plans with FP64 butterflies
+constexpr DefaultVariant kDefaultXp[] = {
+    {ROLE_T_X_FWD, 256, "r16x16/E16/xp/G16/full/wide"},         // first 1.11, 1.15
+    {ROLE_T_X_FWD, 512, "r8x8x8/E8/xp/G16/split/wide/nt"},      // 1.02
+    {ROLE_T_X_FWD, 1024, "r16x16x4/E16/xp/G8/split/wide"},      // 1.13
+    {ROLE_T_Y_FWD, 128, "r16x8/E16/xp/G16/split/wide1"},        // 1.07
+    {ROLE_T_Y_FWD, 256, "r16x16/E16/xp/G16/split/wide2/nt"},    // 1.11
+    {ROLE_T_Y_FWD, 512, "r8x8x8/E8/xp/G16/split/wide2/nt"},     // 1.00, 1.12
+    {ROLE_T_Y_FWD, 1024, "r16x16x4/E16/xp/G16/split/wide2/nt"}, // (as 256)
+    {ROLE_T_Z, 128, "r8x4x4/E8/xp/G4/full/mt"},                 // 1.06
+    {ROLE_T_Z, 256, "r16x16/E16/xp/G4/split/mt"},               // 1.31
+    {ROLE_T_Z, 512, "r8x8x8/E8/xp/G1/full/mt"},                 // 1.13
+    {ROLE_T_Z, 1024, "r16x16x4/E16/xp/G2/split/mtp"},           // 1.2
+    {ROLE_T_Y_INV, 128, "r8x4x4/E8/xp/G16/split/wide2/nt"},     // 1.13
+    {ROLE_T_Y_INV, 256, "r16x16/E16/xp/G16/split/wide2/nt"},    // 1.08 (in a run)
+    {ROLE_T_Y_INV, 512, "r16x16x2/E16/xp/G16/split/wide2"},     // 1.00, 1.06
+    {ROLE_T_Y_INV, 1024, "r16x16x4/E16/xp/G16/split/wide2"},
+    {ROLE_T_X_INV, 128, "r16x8/E16/xp/G16"},                    // 1.09 (in a run)
+    {ROLE_T_X_INV, 256, "r16x16/E16/xp/G16"}};                  // 1.05
+// z pass of PFC plans whose three run spectra fit the last-level cache
+constexpr DefaultVariant kCachedZF64[] = {{ROLE_T_Z, 128, "r8x4x4/E8/G4/full"},
+                                          {ROLE_T_Z, 256, "r16x16/E16/G4/split"},
+                                          {ROLE_T_Z, 512, "r8x8x8/E8/G1/split/pre"}};
+constexpr DefaultVariant kCachedZF32[] = {{ROLE_T_Z, 128, "r16x8/E16/G8/full"},
+                                          {ROLE_T_Z, 256, "r8x8x4/E8/G2/full"},
+                                          {ROLE_T_Z, 512, "r8x8x8/E8/G2/split"}};
+
+template <typename T>
+void pick_variants(pfc_hip_plan_s *p, const DefaultVariant *d, size_t count) {
+  for (size_t i = 0; i < count; ++i) {
+    if (p->role_len(d[i].role) != d[i].n) continue;
+    const int nv = variant_count<T>(p, d[i].role);
+    for (int v = 0; v < nv; ++v)
+      if (*variant_name<T>(p, d[i].role, v) == d[i].name) p->var[d[i].role] = v;
+  }
+}
+
+// The transposed z pass depends on the model too, which the operators set: the
+// table forms mark their lines non-temporal, which is right where the next pass
+// finds them in HBM anyway and wrong for a PFC run whose three spectra (A2, B2,
+// A1) the 256 MB last-level cache holds.  ms per step of a run, plain lines
+// against the table form: FP32 256^3 .129 / .137, 256x256x128 .076 / .085,
+// 256x128x512 .140 / .145, FP64 256x128x128 .070 / .075; beyond the cache FP32
+// 256x256x512 (3 x 135 MB) .254 / .250.  Tungsten's multipliers cost more than
+// the lines: the table form is ahead at every size (FP64 256x128x128 .141).
+constexpr size_t kLastLevelCache = 256u << 20;
+template <typename T> void default_z(pfc_hip_plan_s *p) {
+  if (!p->z_default || p->xp || !p->t_ok) return;
+  const bool cached = 3 * p->outbox() * 2 * p->esize <= kLastLevelCache && !p->tungsten();
+  if (cached && sizeof(T) == 8)
+    pick_variants<T>(p, kCachedZF64, std::size(kCachedZF64));
+  else if (cached)
+    pick_variants<T>(p, kCachedZF32, std::size(kCachedZF32));
+  else
+    for (const DefaultVariant &d : kDefaultF64)
+      if (d.role == ROLE_T_Z && sizeof(T) == 8) pick_variants<T>(p, &d, 1);
+  if (!cached && sizeof(T) == 4)
+    for (const DefaultVariant &d : kDefaultF32)
+      if (d.role == ROLE_T_Z) pick_variants<T>(p, &d, 1);
+}
+
 // The variant each role of a new plan starts with.
 template <typename T> void default_variants(pfc_hip_plan_s *p) {
+  if (p->xp)
+    pick_variants<T>(p, kDefaultXp, std::size(kDefaultXp));
+  else if (sizeof(T) == 8)
+    pick_variants<T>(p, kDefaultF64, std::size(kDefaultF64));
+  else
+    pick_variants<T>(p, kDefaultF32, std::size(kDefaultF32));
   for (int r = 0; r < ROLE_COUNT; ++r)
     if (plane_role(r) && row_variant_count<T>(p, r) > 0 && plane_variant_default(p))
       p->var[r] = row_variant_count<T>(p, r);
@@ -1409,6 +1562,10 @@ int pfc_hip_pfc_set_operators(pfc_hip_plan_t plan, int model_kind,
     plan->tq[4] = params[10];                                  // stabP
   }
   plan->model_kind = model_kind;
+  if (plan->prec == PFC_HIP_F64)
+    default_z<double>(plan);
+  else
+    default_z<float>(plan);
   if (int rc = step_buffers(plan)) return rc;
   plan->dt = dt;
   plan->ops_ready = true;
@@ -1965,6 +2122,7 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index) {
   }
   if (plan->var[role] != index) ++plan->gen;
   plan->var[role] = index;
+  if (role == ROLE_T_Z) plan->z_default = false;
   if ((role == ROLE_STEP_LAYOUT || plane_role(role)) && plan->ops_ready)
     return step_buffers(plan);
   return 0;
@@ -2204,7 +2362,15 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
     }
     // a batched plan's transposed step times its field 0 (the fields run
     // one after another); the natural one times every field at once
-    layout_ms[layout] = layout == 0 ? fastest * plan->batch : fastest;
+    if (layout == 0) fastest *= plan->batch;
+    // multi-step runs, where they are faster than single steps (a run covers
+    // every field of the plan)
+    constexpr int kLayoutRun = 6;
+    for (int r = 0; r <= reps && !rc && !plan->tungsten(); ++r) {
+      const double ms = run_ms_of(kLayoutRun) / kLayoutRun;
+      if (r > 0) fastest = std::min(fastest, ms);
+    }
+    layout_ms[layout] = fastest;
   }
   if (!rc && two) {
     rc = pfc_hip_variant_set(plan, ROLE_STEP_LAYOUT,
@@ -2217,6 +2383,7 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
   ++plan->gen; // the variants of every tuned role may have changed
+  plan->z_default = false;
   // psi is restored on every exit path once the backup was enqueued; a
   // failure of the sweep keeps its own code and message
   const std::string sweep_error = rc ? g_last_error : std::string();

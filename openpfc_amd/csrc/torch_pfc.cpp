@@ -74,6 +74,15 @@ pfc_hip_plan_t plan_for(int nx, int ny, int nz, int prec) {
     // a state recomputed from a checkpoint has to be the state of the forward
     // run bit for bit, however many steps a call takes
     check(pfc_hip_variant_set(p->h, PFC_HIP_ROLE_STEP_FUSE, 0), "pfc_trajectory: single steps");
+    // The FP32-mixed trajectory returns FP64 tensors that carry FP32 rounding: it
+    // stays on the first variant of every pass, so that its results do not move
+    // with the defaults picked for speed.
+    for (int r = 0; prec == PFC_HIP_F32 && r < PFC_HIP_ROLE_COUNT; ++r) {
+      int count = 0;
+      check(pfc_hip_variant_count(p->h, r, &count), "pfc_trajectory: variants");
+      if (count > 0 && r != PFC_HIP_ROLE_STEP_LAYOUT)
+        check(pfc_hip_variant_set(p->h, r, 0), "pfc_trajectory: variants");
+    }
   }
   return p->h;
 }
