@@ -46,7 +46,7 @@ def _run(cmd, quiet=True):
 SOURCES = ["pfc_hip.hip", "variants_common.hip", "variants_f64.hip", "variants_f32.hip",
            "variants_tx_f64.hip", "variants_ty_f64.hip", "variants_tz_f64.hip",
            "variants_tx_f32.hip", "variants_ty_f32.hip", "variants_tz_f32.hip",
-           "variants_t_xp.hip", "plane_f64.hip", "plane_f32.hip", "field_io.hip",
+           "variants_t_xp.hip", "plane_f64.hip", "plane_f32.hip", "adjoint_f64.hip", "field_io.hip",
            "ensemble.hip"]
 OBJDIR = os.path.join(HERE, "_build")
 

@@ -20,33 +20,9 @@
 // k = 0, where dopL = dopN = 0.
 #pragma once
 
-#include "fft_kernels.hpp"
+#include "adjoint_z.hpp"
 
 namespace pfc_amd {
-
-// d opL / d eps and d opN / d eps for one mode (unscaled).
-__device__ __forceinline__ void pfc_op_deriv(const PfcOp &o, double kxy, double kz,
-                                             double &opL, double &opN, double &dL,
-                                             double &dN) {
-#pragma clang fp contract(off)
-  const double k2 = (kxy + (kz * kz));
-  const double k2_lap = -k2;
-  const double one_m = 1.0 - k2;
-  const double L = (k2_lap * (o.eps + (one_m * one_m)));
-  const double oL = exp((L * o.dt));
-  opL = oL;
-  if (fabs(L) > 1e-14) {
-    opN = ((oL - 1.0) / L * k2_lap);
-    // dt*opL*L - (opL - 1) = x e^x - expm1(x), x = L dt
-    const double x = L * o.dt;
-    const double num = (x * oL) - expm1(x);
-    dN = ((k2_lap * k2_lap) * num) / (L * L);
-  } else {
-    opN = (o.dt * k2_lap);
-    dN = 0.0;
-  }
-  dL = (o.dt * k2_lap) * oL;
-}
 
 // n3 = psi^3 (the reference's psi*psi*psi), or psi^3 - m^3 from the
 // deviation (Nonlin of the forward step)
