@@ -49,6 +49,13 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n) {
   }
 }
 
+// The same order with runs of P = 2^lg consecutive blocks per XCD.
+__device__ __forceinline__ unsigned xcd_runs(unsigned b, unsigned n, int lg) {
+  if (b >= (n >> (lg + 3) << (lg + 3))) return b;
+  const unsigned x = b & 7u, r = b >> 3;
+  return (((r >> lg) * 8 + x) << lg) + (r & ((1u << lg) - 1));
+}
+
 // ----------------------------------------------------------------------------
 // Column transform along y or z.
 //   column (x, outer) starts at outer*s_outer + x; position p at + p*s_pos.
@@ -62,6 +69,7 @@ template <typename T> struct ColArgs {
   long s_outer;
   int W;   // active columns in x
   int ntx; // tiles in x
+  int lg;  // log2 of the consecutive tiles an XCD runs (xcd_run_log2)
 };
 
 template <typename T, typename Plan, int DIR, int L, bool SPLIT>
@@ -76,7 +84,7 @@ __global__ void __launch_bounds__(L *Plan::TL)
   const cplx<T> *__restrict__ src = a.src[f];
   cplx<T> *__restrict__ dst = a.dst[f];
   const int c = threadIdx.x % L, t = threadIdx.x / L;
-  const unsigned bid = xcd_block<T, L>(blockIdx.x, gridDim.x);
+  const unsigned bid = xcd_runs(blockIdx.x, gridDim.x, a.lg);
   const int tx = (int)(bid % (unsigned)a.ntx);
   const long outer = bid / (unsigned)a.ntx;
   const int x = tx * L + c;

@@ -123,7 +123,7 @@ struct pfc_hip_plan_s {
   void *A = nullptr, *B = nullptr;
   void *C = nullptr; // natural layout with plane kernels: Psi between x/y and z
   void *A1 = nullptr, *B1 = nullptr, *A2 = nullptr, *B2 = nullptr;
-  // adjoint workspace: three outbox spectra, two real fields, block partials
+  // adjoint workspace: three spectra (of pitch P at most), two real fields, block partials
   void *adj_lam = nullptr, *adj_P = nullptr, *adj_N = nullptr;
   void *adj_a = nullptr, *adj_b = nullptr, *adj_part = nullptr;
   void *adj_zpart = nullptr; // block partials of the fused z pass
@@ -1070,11 +1070,11 @@ int sum_partials(double *part, int n, double *out, hipStream_t s) {
 // spectral part in one pass (k_adj_z): x and y passes of psi, N(psi) and lambda
 // (one plane launch where the plane kernels are on), k_adj_z, inverse y and x with
 // the combine (one plane launch).  128^3 FP64: 33 + 33 + 31 us and the reduction's 6,
-// against 13 launches of 187 us pass by pass; 20 steps forward and back 4.35 ms
+// against 13 launches of 187 us pass by pass; 20 steps forward and back 4.24 ms
 // (6.33 before).
 int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hipStream_t s) {
   using T = double;
-  const size_t cb = p->outbox() * 2 * p->esize, rb = p->inbox() * p->esize;
+  const size_t cb = p->padded() * 2 * p->esize, rb = p->inbox() * p->esize;
   const int blocks = adj_z_blocks(p->W, p->ny, p->nz);
   const bool pf = on_plane<T>(p, ROLE_PFC_X), pi = on_plane<T>(p, ROLE_X_C2R);
   int rc = 0;
@@ -1089,7 +1089,7 @@ int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
   // lambda takes the same kernel with and without dr: same bits
   const bool all = dr && pf && on_plane<T>(p, ROLE_X_R2C);
   if (dr && pf) {
-    PlaneArgs<T> a = plane_args<T>(p, p->W);
+    PlaneArgs<T> a = plane_args<T>(p, p->P);
     a.psi_in = (const T *)psi;
     a.lam_in = (const T *)lambda;
     a.dst[0] = (cplx<T> *)p->adj_P;
@@ -1098,9 +1098,9 @@ int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
     a.nfields = all ? 3 : 2;
     PFC_HIP_TRY(plane_pass<T>(p, PL_FWD, a, s), "adjoint forward plane pass");
   } else if (dr) {
-    if ((rc = pfc_xy_rows<T>(p, psi, p->adj_P, p->adj_N, p->W, s))) return rc;
+    if ((rc = pfc_xy_rows<T>(p, psi, p->adj_P, p->adj_N, p->P, s))) return rc;
   }
-  if (!all && (rc = r2c_xy<T>(p, lambda, p->adj_lam, p->W, s))) return rc;
+  if (!all && (rc = r2c_xy<T>(p, lambda, p->adj_lam, p->P, s))) return rc;
   AdjZArgs z{};
   z.lam = (const cplx<T> *)p->adj_lam;
   z.P = (cplx<T> *)p->adj_P;
@@ -1108,13 +1108,13 @@ int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
   z.tw = twp<T>(p, p->nz, adj_z_plan(p->nz));
   z.op = p->op;
   z.partial = (double *)p->adj_zpart;
-  z.s_pos = (long)p->W * p->ny;
-  z.pitch = p->W;
+  z.s_pos = (long)p->P * p->ny;
+  z.pitch = p->P;
   z.W = p->W;
   z.want_dr = dr ? 1 : 0;
   PFC_HIP_TRY(adj_z_launch(z, s), "adjoint z pass");
   if (pi) {
-    PlaneArgs<T> a = plane_args<T>(p, p->W);
+    PlaneArgs<T> a = plane_args<T>(p, p->P);
     a.src = (const cplx<T> *)p->adj_P;
     a.src2 = (const cplx<T> *)p->adj_N;
     a.psi_in = (const T *)psi;
@@ -1123,10 +1123,10 @@ int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
     PFC_HIP_TRY(plane_pass<T>(p, PL_ADJ, a, s), "adjoint inverse plane pass");
   } else {
     if (p->ny > 1)
-      PFC_HIP_TRY(col_pass<T>(p, 1, +1, p->adj_P, p->adj_P, p->adj_N, p->adj_N, 2, p->W, s),
+      PFC_HIP_TRY(col_pass<T>(p, 1, +1, p->adj_P, p->adj_P, p->adj_N, p->adj_N, 2, p->P, s),
                   "adjoint inverse y pass");
-    PFC_HIP_TRY(x_c2r_pass<T>(p, p->adj_P, p->adj_a, p->W, 1.0, s), "adjoint inverse x pass");
-    PFC_HIP_TRY(x_c2r_pass<T>(p, p->adj_N, p->adj_b, p->W, 1.0, s), "adjoint inverse x pass");
+    PFC_HIP_TRY(x_c2r_pass<T>(p, p->adj_P, p->adj_a, p->P, 1.0, s), "adjoint inverse x pass");
+    PFC_HIP_TRY(x_c2r_pass<T>(p, p->adj_N, p->adj_b, p->P, 1.0, s), "adjoint inverse x pass");
     const long n = (long)p->inbox();
     hipLaunchKernelGGL(k_adj_combine<T>, dim3(ic_blocks(n)), dim3(256), 0, s, (const T *)psi,
                        (const T *)p->adj_a, (const T *)p->adj_b, (T *)lambda, n, mean);
@@ -1144,7 +1144,7 @@ int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
 // returns FP64 tensors that carry the FP32 rounding of exactly these passes.
 int adjoint_f32(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hipStream_t s) {
   using T = float;
-  const size_t cb = p->outbox() * 2 * p->esize, rb = p->inbox() * p->esize;
+  const size_t cb = p->padded() * 2 * p->esize, rb = p->inbox() * p->esize;
   int rc = 0;
   if (!rc) rc = dalloc(p, &p->adj_lam, cb, "adjoint spectrum");
   if (!rc) rc = dalloc(p, &p->adj_P, cb, "adjoint spectrum");
@@ -1185,7 +1185,7 @@ int adjoint_f32(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hi
 // Free energy of the plain PFC model (energy_kernels.hpp), summed in double.
 template <typename T>
 int free_energy_impl(pfc_hip_plan_s *p, const void *psi, double *F, hipStream_t s) {
-  int rc = dalloc(p, &p->adj_P, p->outbox() * 2 * p->esize, "free-energy spectrum");
+  int rc = dalloc(p, &p->adj_P, p->padded() * 2 * p->esize, "free-energy spectrum");
   if (!rc) rc = dalloc(p, &p->adj_part, kPartials * sizeof(double), "reduction partials");
   if (rc) return rc;
   if ((rc = r2c_impl<T>(p, psi, p->adj_P, s))) return rc;

@@ -10,7 +10,7 @@ namespace pfc_amd {
 // PL_INV  src -> psi_out * scale
 // PL_BND  src -> psi in registers -> blockIdx.y = 0: psi, 1: N(psi) -> dst
 // PL_TUNG src (mean field) -> N(psi_in, mean field) -> dst[0]; optional mf_out
-// PL_ADJ  src, src2 -> a, b in real space; psi_out = a + 3 (m + psi_in)^2 b
+// PL_ADJ  src, src2 -> a, b in real space; psi_out = a + 3 (m + psi_in)^2 b (double)
 enum PlaneMode { PL_FWD = 0, PL_INV = 1, PL_BND = 2, PL_TUNG = 3, PL_ADJ = 4 };
 
 template <typename T> struct PlaneArgs {

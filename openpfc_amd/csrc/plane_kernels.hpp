@@ -286,15 +286,17 @@ hipError_t plane_launch_mode(const PlaneArgs<T> &a, long planes, hipStream_t s) 
     case PL_INV: return plane_launch_mode<T, PL_INV>(a, planes, s);                         \
     case PL_BND: return plane_launch_mode<T, PL_BND>(a, planes, s);                         \
     case PL_TUNG: return plane_launch_mode<T, PL_TUNG>(a, planes, s);                       \
-    case PL_ADJ: return plane_launch_mode<T, PL_ADJ>(a, planes, s);                         \
+    case PL_ADJ:                                                                            \
+      if constexpr (sizeof(T) == 8) return plane_launch_mode<T, PL_ADJ>(a, planes, s);      \
+      [[fallthrough]];                                                                      \
     default: return hipErrorInvalidValue;                                                   \
     }                                                                                       \
   }                                                                                         \
   template <> hipError_t plane_init<T>() {                                                  \
     for (hipError_t e : {plane_init_mode<T, PL_FWD>(), plane_init_mode<T, PL_INV>(),        \
-                         plane_init_mode<T, PL_BND>(), plane_init_mode<T, PL_TUNG>(),       \
-                         plane_init_mode<T, PL_ADJ>()})                                     \
+                         plane_init_mode<T, PL_BND>(), plane_init_mode<T, PL_TUNG>()})      \
       if (e != hipSuccess) return e;                                                        \
+    if constexpr (sizeof(T) == 8) return plane_init_mode<T, PL_ADJ>();                      \
     return hipSuccess;                                                                      \
   }
 
