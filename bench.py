@@ -95,9 +95,12 @@ def variant_key(kernel, prec, n, variant, direction=None, mode=0):
         wpe = pb[4][1:] if len(pb) > 4 and pb[4][:1] == "w" else "1"  # waves per SIMD cap
         return (f"k_tx_fuse<{t},N{n // 2}/E{ea[1:]},r{ra[1:]}+N{n}/E{pb[1][1:]},r{pb[0][1:]},"
                 f"{pb[2][1:]},{'true' if pb[3] == 'split' else 'false'},{wpe}>")
-    if kernel == "k_tx_bnd":  # "rA/EA/G8[/wN][/nt]": the nx/2-point plan, both directions
+    if kernel == "k_tx_bnd":  # "rA/EA/G8[/cols][/wN][/nt]": the nx/2-point plan, both directions
         parts = variant.split("/")
         wpe = [p[1:] for p in parts if p[:1] == "w"] or ["1"]
+        if "cols" in parts:
+            return (f"k_tx_cols<{t},N{n // 2}/E{parts[1][1:]},r{parts[0][1:]},{parts[2][1:]},"
+                    f"{wpe[0]},{'true' if 'nt' in parts else 'false'}>")
         return (f"k_tx_bnd<{t},N{n // 2}/E{parts[1][1:]},r{parts[0][1:]},{parts[2][1:]},{wpe[0]},"
                 f"{'true' if 'nt' in parts else 'false'}>")
     parts = variant.split("/")

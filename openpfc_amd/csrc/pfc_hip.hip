@@ -1292,9 +1292,9 @@ constexpr DefaultVariant kDefaultF64[] = {
     {ROLE_T_X_INV, 128, "r8x4x4/E8/G8/nt"},                 // 1.01 to 1.25
     {ROLE_T_X_INV, 256, "r8x8x4/E8/G8/nt"},                 // 1.04 to 1.19
     {ROLE_T_X_INV, 512, "r16x16x2/E16/G8/nt"},              // 1.03, 1.07
-    {ROLE_T_X_FUSE, 128, "r8x4x4/E8/G8/w4"},                // 1.00 to 1.09
-    {ROLE_T_X_FUSE, 256, "r8x8x4/E8/G8/w4"},                // 1.07, 1.09
-    {ROLE_T_X_FUSE, 512, "r16x16x2/E16/G8/w2"},             // 1.04, 1.06
+    {ROLE_T_X_FUSE, 128, "r8x4x4/E8/G8/cols/w4"},           // 1.08
+    {ROLE_T_X_FUSE, 256, "r16x16/E16/G8/cols/w2"},          // 1.17
+    {ROLE_T_X_FUSE, 512, "r8x8x8/E8/G8/cols/w4"},           // 1.20
     {ROLE_T_X_R2C, 128, "r8x4x4/E8/G8"},                    // 1.06, 1.10
     {ROLE_T_X_TUNG, 128, "r8x4x4/E8/G8/wide"},              // 1.05, 1.15
     {ROLE_T_X_TUNG, 256, "r8x8x4/E8/G8/wide/w4"},           // 1.04

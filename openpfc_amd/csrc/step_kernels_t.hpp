@@ -1160,4 +1160,70 @@ __global__ void __launch_bounds__(G *Plan::TL, WPE) k_tx_bnd(TStepArgs<T> a) {
                                [&](int kx, int gg) { return spec + ((long)kx * a.ny + gg); });
 }
 
+// ----------------------------------------------------------------------------
+// The same pass with the block's threads across the tile, G adjacent y at G
+// neighbouring lanes: a spectrum value goes straight from its line to the register
+// the transform wants it in and back, so there is no staging tile to fill and
+// empty (two of the five trips through the LDS) and no wait for the whole
+// tile before the first merge.  The rows' exchanges become block-wide.  In
+// double the eight values of a 128-byte line fill 8 lanes and every plan of 8 or
+// 16 values a thread fits its registers: 4.09 ms against 4.68 at 1024^3, 0.476
+// against 0.518 at 512^3, 68 against 74 us at 256^3 (a whole step of a run 17.60
+// against 18.13, 1.971 against 2.008, 0.242 against 0.245 ms; with non-temporal
+// lines 17.68, 1.970, and up to 5 % slower where the cache holds the step).  In single precision
+// 16 lines of 16 values spill or run few waves (0.323 against 0.324 ms at 512^3,
+// 3.1 against 2.4 at 1024^3): built for double only.  One component at
+// a time (half the LDS, twice the blocks) spilled at the registers those blocks
+// leave: 11.4 ms at 1024^3.  The Tungsten x pass in this form read psi in 128-byte
+// pieces and lost: 0.350 against 0.341 ms at 512x512x256.
+// ----------------------------------------------------------------------------
+template <typename T, typename Plan, int G, int WPE, bool NT>
+__global__ void __launch_bounds__(G *Plan::TL, WPE) k_tx_cols(TStepArgs<T> a) {
+  constexpr int TL = Plan::TL, E = Plan::E, M = Plan::N, NP = row_padded(M);
+  __shared__ T lds[2 * G * NP];
+  const int g = threadIdx.x % G, t = threadIdx.x / G;
+  const int ngy = (a.ny + G - 1) / G;
+  const unsigned bid = xcd_block<T, G>(blockIdx.x, gridDim.x);
+  const int z = (int)bid / ngy, y = ((int)bid % ngy) * G + g;
+  const bool active = y < a.ny;
+  cplx<T> *__restrict__ spec = a.A1 + (long)z * a.W * a.ny + (active ? y : 0);
+  const LdsLine<T> ll{lds, g, G, G * NP};
+  // f(e, value at the mirror position: M - k, or 0 for k = 0) for every e
+  auto with_mirror = [&](const cplx<T>(&v)[E], auto f) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = ll.idx(pad_pos<true>(t + TL * e));
+      lds[i] = v[e].x;
+      lds[i + G * NP] = v[e].y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int k = t + TL * e;
+      const int i = ll.idx(pad_pos<true>(k == 0 ? 0 : M - k));
+      f(e, cplx<T>{lds[i], lds[i + G * NP]});
+    }
+    __syncthreads(); // the area is free again
+  };
+
+  cplx<T> v[E], xm{};
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = ld_line<NT>(&spec[(long)(t + TL * e) * a.ny]);
+  if (t == 0) xm = ld_line<NT>(&spec[(long)M * a.ny]);
+  with_mirror(v, [&](int e, cplx<T> p) {
+    const int k = t + TL * e;
+    v[e] = c2r_merge(v[e], k == 0 ? xm : p, a.wn[k], k == 0);
+  });
+  LineFft<T, Plan, +1, false, true>::run(v, t, ll, a.tw_xm);
+#pragma unroll
+  for (int e = 0; e < E; ++e) v[e] = cplx<T>{a.nl(v[e].x), a.nl(v[e].y)};
+  LineFft<T, Plan, -1, false, true>::run(v, t, ll, a.tw_xm);
+  xm = cplx<T>{v[0].x - v[0].y, (T)0}; // X[M], on t == 0
+  with_mirror(v, [&](int e, cplx<T> p) { v[e] = r2c_split(v[e], p, a.wn[t + TL * e]); });
+  if (!active) return;
+#pragma unroll
+  for (int e = 0; e < E; ++e) st_line<NT>(&spec[(long)(t + TL * e) * a.ny], v[e]);
+  if (t == 0) st_line<NT>(&spec[(long)M * a.ny], xm);
+}
+
 } // namespace pfc_amd

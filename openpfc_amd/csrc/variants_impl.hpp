@@ -501,6 +501,13 @@ hipError_t tx_bnd_launch(TStepArgs<T> a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename T, typename Plan, int G, int WPE, bool NT>
+hipError_t tx_cols_launch(TStepArgs<T> a, hipStream_t s) {
+  dim3 grid((unsigned)(a.nz * ((a.ny + G - 1) / G))), block(G * Plan::TL);
+  hipLaunchKernelGGL((k_tx_cols<T, Plan, G, WPE, NT>), grid, block, 0, s, a);
+  return hipGetLastError();
+}
+
 template <typename T, typename Plan, int G, bool S, int NR, bool NT = false>
 hipError_t ty_fwd_w_launch(TStepArgs<T> a, hipStream_t s) {
   if (a.nfields != 1 && a.nfields != 2) return hipErrorInvalidValue;
@@ -647,6 +654,19 @@ void add_t_bnd(std::vector<TV<T>> &v, int pid) {
                      (WPE > 1 ? "/w" + std::to_string(WPE) : "") + (NT ? "/nt" : ""),
                  pid, &tx_bnd_launch<T, Plan, G, WPE, NT>});
 }
+// The boundary pass with threads across the tile (double only, see k_tx_cols);
+// registers capped so that the blocks the LDS allows all fit, at 128 of them
+// at least
+template <typename T, typename Plan, int G, bool NT> void add_t_cols(std::vector<TV<T>> &v, int pid) {
+  constexpr int lds = 2 * G * row_padded(Plan::N) * (int)sizeof(T), nw = G * Plan::TL / 64;
+  if constexpr (sizeof(T) == 8 && Plan::E >= 8 && nw >= 1 && nw <= kMaxThreads / 64 &&
+                lds <= kMaxLds) {
+    constexpr int fit = 160 * 1024 / lds * nw / 4, wpe = fit > 4 ? 4 : fit < 1 ? 1 : fit;
+    v.push_back({plan_name<Plan>() + "/G" + std::to_string(G) + "/cols/w" + std::to_string(wpe) +
+                     (NT ? "/nt" : ""),
+                 pid, &tx_cols_launch<T, Plan, G, wpe, NT>});
+  }
+}
 // Tungsten fused x pass, wide store, registers capped for WPE waves per SIMD
 template <typename T, typename Plan, int G, int WPE>
 void add_t_tung_wide_o(std::vector<TV<T>> &v, int pid) {
@@ -751,6 +771,8 @@ template <typename T, int N, int KIND> std::vector<TV<T>> make_t_kind() {
           add_t_bnd<T, P, G0, wpe>(v, pid);
           add_t_bnd<T, P, G0, wpe, true>(v, pid);
         }
+        add_t_cols<T, P, G0, false>(v, pid);
+        add_t_cols<T, P, G0, true>(v, pid);
       });
     }
     if constexpr (KIND == TK_X_R2C || KIND == TK_X_TUNG) {
