@@ -270,7 +270,18 @@ hipError_t plane_launch_mode(const PlaneArgs<T> &a, long planes, hipStream_t s) 
   const size_t lds = plane_lds<T>(a.nx, a.ny);
   if (!lds || planes < 1 || planes > 0x7fffffffL) return hipErrorInvalidValue;
   const int nf = (MODE == PL_FWD || MODE == PL_BND) ? a.nfields : 1;
-  const int nt = 64 * plane_waves<T>(a.nx, a.ny);
+  int nt = 64 * plane_waves<T>(a.nx, a.ny);
+  // A CU runs one block of 9 to 16 waves at a time (128 registers a thread), and its
+  // loads, transforms and stores follow each other.  With more blocks than the
+  // 256 CUs, and room in the LDS for two, 8 waves a block let two blocks overlap.
+  // Single precision, us of a step of a run with 16 | 8 waves: 128x128x256
+  // 52.9 | 46.3, 128x128x512 105 | 89, 96x192x512 121 | 103, 256x64x512 96 | 84,
+  // 192x96x512 102 | 98.  At 256 blocks and below both take the same time or
+  // 8 waves lose (128x128x64: 25.5 | 26.4), as they do in the inverse pass alone
+  // (25.5 | 26.2 at 128x128x512); doubles differ by 1 % either way.
+  if constexpr (sizeof(T) == 4 && (MODE == PL_FWD || MODE == PL_BND)) {
+    if (nt > 512 && planes * nf > 256 && 2 * lds <= 160 * 1024) nt = 512;
+  }
   const dim3 grid((unsigned)planes, (unsigned)nf);
   if (nt <= 512)
     hipLaunchKernelGGL((k_plane<T, MODE, 512>), grid, dim3(nt), lds, s, a);
