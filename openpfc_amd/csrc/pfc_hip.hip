@@ -760,7 +760,7 @@ int step_transposed(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev)
 //
 // Measured, ms per step of a run, tuned variants, kept spectrum against psi
 // transformed anew at a fused boundary (12C) and against single steps (12C + 2R):
-//   FP64 1024^3 18.1 / 21.1 / 23.1 (y 3.14, z 5.35, inverse y 3.47, boundary 4.70)
+//   FP64 1024^3 17.6 / 21.1 / 23.1 (y 3.14, z 5.35, inverse y 3.47, boundary 4.09)
 //   FP32 1024^3  9.3 / 11.6 / 12.0 (y 1.60, z 2.76, inverse y 1.75, boundary 2.40)
 //   FP64  512^3 2.00 / 2.50 / 2.75,  FP32 512^3 1.07 / 1.34 / 1.42
 //   FP64  256^3 .245 / .334 / .363,  FP32 256^3 .134 / .156 / .188
@@ -1270,7 +1270,8 @@ constexpr DefaultVariant kDefaultF64[] = {
     {ROLE_X_R2C, 256, "r4x4x4x4/E4/rows1"},            // 1.08
     {ROLE_X_C2R, 128, "r8x4x4/E8/rows16"},             // 1.07 to 1.12
     {ROLE_X_C2R, 256, "r4x4x4x4/E4/rows2"},            // 1.02 to 1.11
-    {ROLE_X_C2R, 512, "r16x16x2/E16/rows4"},           // 1.13
+    // rows of 1024: no line; r16x16x2/E16/rows4 is 2 % ahead from 36864 rows up
+    // (C2R 405 | 414 us) and 2 to 6 % behind below (256 rows 16.5 | 15.7)
     {ROLE_X_TUNG, 128, "r8x4x4/E8/rows4"},             // 1.24, 1.52
     {ROLE_X_TUNG, 256, "r4x4x4x4/E4/rows1"},           // 1.05
     // transposed layout
