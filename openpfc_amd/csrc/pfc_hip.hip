@@ -141,7 +141,7 @@ struct pfc_hip_plan_s {
   bool mean_split = false; // field holds psi - mean; mean kept in double here
   double mean = 0.0;
   int var[ROLE_COUNT] = {};
-  bool z_default = true; // the transposed z variant is still the default's
+  bool chosen[ROLE_COUNT] = {}; // roles set by a caller or the autotuner
   size_t bytes = 0;
   // Batched plans step `batch` fields of these extents stored one after
   // another.  The natural layout steps them all in each launch, reading
@@ -1373,7 +1373,7 @@ void pick_variants(pfc_hip_plan_s *p, const DefaultVariant *d, size_t count) {
 // the lines: the table form is ahead at every size (FP64 256x128x128 .141).
 constexpr size_t kLastLevelCache = 256u << 20;
 template <typename T> void default_z(pfc_hip_plan_s *p) {
-  if (!p->z_default || p->xp || !p->t_ok) return;
+  if (p->chosen[ROLE_T_Z] || p->xp || !p->t_ok) return;
   const bool cached = 3 * p->outbox() * 2 * p->esize <= kLastLevelCache && !p->tungsten();
   if (cached && sizeof(T) == 8)
     pick_variants<T>(p, kCachedZF64, std::size(kCachedZF64));
@@ -1399,6 +1399,26 @@ template <typename T> void default_variants(pfc_hip_plan_s *p) {
     if (plane_role(r) && row_variant_count<T>(p, r) > 0 && plane_variant_default(p))
       p->var[r] = row_variant_count<T>(p, r);
   p->var[ROLE_STEP_FUSE] = variant_count<T>(p, ROLE_STEP_FUSE) - 1;
+}
+
+// Defaults that depend on the model.  A single-precision Tungsten step keeps the
+// first variant of every role: a moving front reads the field's column maxima in
+// double, which carry the FP32 rounding of exactly these passes (others are as
+// accurate, 7.5e-8 against 9.0e-8, but 8e-8 away).
+template <typename T> void model_variants(pfc_hip_plan_s *p) {
+  if (sizeof(T) == 8 || p->xp) {
+    default_z<T>(p);
+    return;
+  }
+  int kept[ROLE_COUNT];
+  std::copy(std::begin(p->var), std::end(p->var), kept);
+  if (p->tungsten())
+    std::fill(std::begin(p->var), std::end(p->var), 0);
+  else
+    default_variants<T>(p);
+  for (int r = 0; r < ROLE_COUNT; ++r)
+    if (p->chosen[r] || r == ROLE_STEP_LAYOUT || r == ROLE_STEP_FUSE) p->var[r] = kept[r];
+  if (!p->tungsten()) default_z<T>(p);
 }
 
 int check_plan(pfc_hip_plan_t p) {
@@ -1657,9 +1677,9 @@ int pfc_hip_pfc_set_operators(pfc_hip_plan_t plan, int model_kind,
   }
   plan->model_kind = model_kind;
   if (plan->prec == PFC_HIP_F64)
-    default_z<double>(plan);
+    model_variants<double>(plan);
   else
-    default_z<float>(plan);
+    model_variants<float>(plan);
   if (int rc = step_buffers(plan)) return rc;
   plan->dt = dt;
   plan->ops_ready = true;
@@ -2216,7 +2236,7 @@ int pfc_hip_variant_set(pfc_hip_plan_t plan, int role, int index) {
   }
   if (plan->var[role] != index) ++plan->gen;
   plan->var[role] = index;
-  if (role == ROLE_T_Z) plan->z_default = false;
+  plan->chosen[role] = true;
   if ((role == ROLE_STEP_LAYOUT || plane_role(role)) && plan->ops_ready)
     return step_buffers(plan);
   return 0;
@@ -2477,7 +2497,7 @@ int pfc_hip_pfc_autotune(pfc_hip_plan_t plan, void *psi, int reps, void *stream,
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
   ++plan->gen; // the variants of every tuned role may have changed
-  plan->z_default = false;
+  std::fill(std::begin(plan->chosen), std::end(plan->chosen), true);
   // psi is restored on every exit path once the backup was enqueued; a
   // failure of the sweep keeps its own code and message
   const std::string sweep_error = rc ? g_last_error : std::string();
