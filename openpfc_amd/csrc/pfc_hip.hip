@@ -1324,8 +1324,7 @@ constexpr DefaultVariant kDefaultF32[] = {
     {ROLE_T_Y_INV, 1024, "r16x16x4/E16/G16/split/wide2"},    // 1.08
     {ROLE_T_X_INV, 512, "r8x8x8/E8/G16/nt"},                 // 1.05, 1.35
     {ROLE_T_X_FUSE, 128, "r16x8/E16/G8"},                    // 1.04, 1.06
-    {ROLE_T_X_FUSE, 512, "r16x16x2/E16/G16/nt"},             // 1.19, 1.29
-    {ROLE_T_X_TUNG, 256, "r16x16/E16/G16/wide"}};            // 1.01
+    {ROLE_T_X_FUSE, 512, "r16x16x2/E16/G16/nt"}};            // 1.19, 1.29
 // plans with FP64 butterflies
 constexpr DefaultVariant kDefaultXp[] = {
     {ROLE_T_X_FWD, 256, "r16x16/E16/xp/G16/full/wide"},         // first 1.11, 1.15
