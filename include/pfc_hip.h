@@ -256,11 +256,13 @@ int pfc_hip_pfc_set_members(pfc_hip_plan_t plan, const double *eps, const double
  * mean-field filter, inverse), 3 inverse-y, 4 x (inverse, N, forward),
  * 5 forward-y, 6 z (forward, combine, inverse), 7 inverse-y, 8 inverse-x.
  * PFC with nkernels >= 6 and nsteps >= 2 where pfc_hip_pfc_step fuses step
- * boundaries: the launches of that fused run, kernel_ms[0] the forward x of
- * the first step, 1..3 the mean y, z and inverse y passes, 4 the inverse x of
- * the last step and 5 the mean fused boundary pass (otherwise kernel_ms[5]
- * = 0).  The means are over the steps after the first, which alone transforms
- * psi too.  No reference counterpart (profiling aid).
+ * boundaries: the launches of that call, which is one run or several (the
+ * spectrum is made anew between them).  kernel_ms[0] is the forward x of a
+ * run's first step, 1..3 the y, z and inverse y passes of the steps after a
+ * run's first (which alone transforms psi too; of all steps where every run
+ * is a single one), 4 the inverse x that ends a run and 5 the fused boundary
+ * pass, each a mean (kernel_ms[5] = 0 where nothing is fused).
+ * No reference counterpart (profiling aid).
  */
 int pfc_hip_pfc_step_timed(pfc_hip_plan_t plan, void *psi, int nsteps,
                            void *stream, double *kernel_ms, int nkernels);

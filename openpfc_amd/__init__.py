@@ -302,10 +302,11 @@ class PfcStepper(_Stepper):
         self.dt = None
 
     def step_timed_fused(self, psi, nsteps: int, stream=None):
-        """The launches of a fused multi-step run (nsteps >= 2): returns
-        [forward x (first step), y forward, z, y inverse (means), inverse x
-        (last step), fused boundary (mean)] in ms; the last entry is 0 when
-        the plan does not fuse step boundaries."""
+        """The launches of step(psi, nsteps), nsteps >= 2, with fused step
+        boundaries: returns the mean ms of [forward x (first step of a run),
+        y forward, z, y inverse (steps after the first), inverse x (end of a
+        run), fused boundary]; the last entry is 0 when the plan does not
+        fuse step boundaries."""
         self._check_psi(psi, "step_timed_fused")
         out = (ctypes.c_double * 6)()
         check(self.fft._lib.pfc_hip_pfc_step_timed(self.fft.handle, _ptr(psi), int(nsteps),

@@ -784,12 +784,17 @@ template <typename T> bool fused_steps(pfc_hip_plan_s *p) {
          !t_list<T>(p, TK_X_FUSE, p->role_len(ROLE_T_X_FUSE)).empty();
 }
 
+// Events steps_fused records for nsteps steps in runs of at most `span`.
+int fused_events(int nsteps, int span) {
+  return 1 + 4 * nsteps + (nsteps + span - 1) / span;
+}
+
 // nsteps >= 1 PFC steps with fused boundaries, in runs of at most fused_span
 // steps: the first step transforms psi and N(psi) (5 passes but the last); the
 // following ones transform N alone (boundary x on T1 of A, forward y A1 -> B2,
 // z with the kept spectrum in A2, inverse y B2 -> A1); the inverse x ends the
-// run.  4*n + 1 launches a run of n.  `ev` (optional) receives 4*nsteps + 2
-// events around the launches of one run of nsteps <= fused_span, in order.
+// run.  4*n + 1 launches a run of n.  `ev` (optional) receives one event before
+// the first launch and one after each, in order: fused_events of them.
 // (Batched plans: the nsteps steps of field 0, then of field 1, ...; `ev`
 // brackets those of field 0.)
 template <typename T>
@@ -800,7 +805,7 @@ int steps_fused(pfc_hip_plan_s *p, void *psi, int nsteps, hipStream_t s, hipEven
       if (ev && m == 0) (void)hipEventRecord(ev[e++], s);
     };
     const TStepArgs<T> a = pfc_t_args<T>(p, psi, m);
-    const int span = ev ? nsteps : fused_span(a.op);
+    const int span = fused_span(a.op);
     mark();
     for (int done = 0; done < nsteps;) {
       const int n = std::min(span, nsteps - done);
@@ -825,9 +830,9 @@ int steps_fused(pfc_hip_plan_s *p, void *psi, int nsteps, hipStream_t s, hipEven
         mark();
       }
       if (int rc = t_pass<T>(p, a, 4, s)) return rc;
+      mark();
       done += n;
     }
-    mark();
   }
   return 0;
 }
@@ -1833,10 +1838,14 @@ int pfc_hip_pfc_step_timed(pfc_hip_plan_t plan, void *psi, int nsteps,
   if (nsteps < 1) return fail(PFC_HIP_EINVAL, "pfc_hip_pfc_step_timed: nsteps < 1");
   hipStream_t s = (hipStream_t)stream;
   const bool f64 = plan->prec == PFC_HIP_F64;
-  // with a sixth entry and a fused run: the launches of pfc_hip_pfc_step
+  // with a sixth entry and a fused run: the launches of pfc_hip_pfc_step, whose
+  // field 0 remakes its spectrum every `span` steps
   const bool fused = nkernels >= 6 && nsteps >= 2 &&
                      (f64 ? fused_steps<double>(plan) : fused_steps<float>(plan));
-  const int ne = fused ? 4 * nsteps + 2 : (np + 1) * nsteps;
+  const int span = !fused ? 1
+                   : f64  ? fused_span(pfc_t_args<double>(plan, psi, 0).op)
+                          : fused_span(pfc_t_args<float>(plan, psi, 0).op);
+  const int ne = fused ? fused_events(nsteps, span) : (np + 1) * nsteps;
   std::vector<hipEvent_t> ev((size_t)ne, nullptr);
   int rc = 0;
   for (auto &e : ev) {
@@ -1862,25 +1871,34 @@ int pfc_hip_pfc_step_timed(pfc_hip_plan_t plan, void *psi, int nsteps,
     hipError_t e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = fail(PFC_HIP_EDEVICE, hipGetErrorString(e));
   }
-  auto span = [&](size_t i) {
+  auto launch_ms = [&](size_t i) {
     float ms = 0;
     (void)hipEventElapsedTime(&ms, ev[i], ev[i + 1]);
     return (double)ms;
   };
   if (!rc && fused) {
-    // launch j of step i is event interval 4*i + j; the exit is 4*nsteps
+    // launch j of step i of a run is the run's interval 4*i + j; its exit the last.
+    // Steps after the first of their run are alike; runs of one step have none.
+    const int runs = (nsteps + span - 1) / span;
+    const int steady = nsteps - runs, first = steady ? 1 : 0, nmid = steady ? steady : nsteps;
     for (int k = 0; k < 6; ++k) kernel_ms[k] = 0;
-    kernel_ms[0] = span(0);
-    for (int i = 1; i < nsteps; ++i) {
-      kernel_ms[5] += span((size_t)4 * i) / (nsteps - 1);
-      for (int k = 1; k <= 3; ++k) kernel_ms[k] += span((size_t)4 * i + k) / (nsteps - 1);
+    size_t base = 0;
+    for (int done = 0; done < nsteps;) {
+      const int n = std::min(span, nsteps - done);
+      kernel_ms[0] += launch_ms(base) / runs;
+      for (int i = first; i < n; ++i) {
+        if (i > 0) kernel_ms[5] += launch_ms(base + 4 * i) / steady;
+        for (int k = 1; k <= 3; ++k) kernel_ms[k] += launch_ms(base + 4 * i + k) / nmid;
+      }
+      kernel_ms[4] += launch_ms(base + 4 * n) / runs;
+      base += 4 * n + 1;
+      done += n;
     }
-    kernel_ms[4] = span((size_t)4 * nsteps);
   } else if (!rc) {
     const int pe = np + 1;
     for (int k = 0; k < np; ++k) kernel_ms[k] = 0;
     for (int i = 0; i < nsteps; ++i)
-      for (int k = 0; k < np; ++k) kernel_ms[k] += span((size_t)pe * i + k) / nsteps;
+      for (int k = 0; k < np; ++k) kernel_ms[k] += launch_ms((size_t)pe * i + k) / nsteps;
     if (nkernels > np) kernel_ms[np] = 0;
   }
   for (auto &e : ev)
