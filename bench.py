@@ -85,7 +85,7 @@ NT_KERNELS = ("k_tz", "k_tx_inv", "k_tx_fwd_w", "k_ty_fwd_w", "k_ty_inv_w")
 def variant_key(kernel, prec, n, variant, direction=None, mode=0):
     """rocprof short name (openpfc_amd.profile_summary.short_name) of a variant;
     `mode` is the z-pass kind (0 PFC, 1 Tungsten mean field, 2 Tungsten combine,
-    3 PFC with the kept spectrum)."""
+    3 PFC with the kept spectrum, 4 PFC keeping its spectrum)."""
     import re
     t = "double" if prec == "f64" else "float"
     if kernel == "k_tx_fuse":  # "rA/EA+rB/EB/G8/split[/wN]": nx/2- and nx-point plans

@@ -519,16 +519,17 @@ template <typename T> struct TungNl {
 // pass): forward N, combine with the kept spectrum, inverse.  ZM_KEEP (PFC
 // runs on the transposed layout that keep Psi's spectrum between steps): the
 // same with the PFC multipliers, the combined spectrum kept in turn.
-enum ZMode { ZM_PFC = 0, ZM_TMF = 1, ZM_TCOMB = 2, ZM_KEEP = 3 };
+// ZM_FIRST (first step of such a run): ZM_PFC with the combined spectrum kept.
+enum ZMode { ZM_PFC = 0, ZM_TMF = 1, ZM_TCOMB = 2, ZM_KEEP = 3, ZM_FIRST = 4 };
 
 // Multipliers of one mode for a z pass of kind MODE, scaled by o.scale:
-// (opL, opN) for ZM_PFC (ZM_KEEP: opL unscaled, since A carries the scale of the
-// step that kept it), (fMF, -) for ZM_TMF, (expL, nW) for ZM_TCOMB.
+// (opL, opN) for ZM_PFC and ZM_FIRST (ZM_KEEP: opL unscaled, since A carries the
+// scale of the step that kept it), (fMF, -) for ZM_TMF, (expL, nW) for ZM_TCOMB.
 template <int MODE>
 __device__ __forceinline__ void z_mode_ops(const PfcOp &o, const TungOp &p,
                                            double kxy, double kz, double &ma,
                                            double &mb) {
-  if constexpr (MODE == ZM_PFC) {
+  if constexpr (MODE == ZM_PFC || MODE == ZM_FIRST) {
     pfc_op_mode(o, kxy, kz, ma, mb);
   } else if constexpr (MODE == ZM_KEEP) {
     PfcOp u = o;

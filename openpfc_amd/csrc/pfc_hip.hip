@@ -816,8 +816,8 @@ int steps_fused(pfc_hip_plan_s *p, void *psi, int nsteps, hipStream_t s, hipEven
           f.A2 = a.B2;
         }
         TStepArgs<T> z = a;
-        z.mode = i > 0 ? ZM_KEEP : ZM_PFC;
         z.keep = i + 1 < n;
+        z.mode = i > 0 ? ZM_KEEP : z.keep ? ZM_FIRST : ZM_PFC;
         TStepArgs<T> y = a; // inverse y
         if (i > 0 || z.keep) y.A2 = a.B2;
         if (int rc = t_pass<T>(p, a, i == 0 ? 0 : 5, s)) return rc;

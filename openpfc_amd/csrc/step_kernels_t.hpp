@@ -89,7 +89,7 @@ __device__ __forceinline__ void fetch_partner(const cplx<T> (&v)[E], cplx<T> (&p
 template <typename T> struct TStepArgs {
   Nonlin<T> nl;     // nonlinearity (plain or mean-split)
   int zero_k0;      // mean-split step: keep the k = 0 mode of the deviation at 0
-  int keep;         // z pass: store the combined spectrum in A2, its inverse in B2
+  int keep;         // ZM_KEEP: store the combined spectrum in A2 too
   int mode;         // k_tz kind (ZMode)
   int nfields;      // k_ty_fwd: 2 (A and B) or 1 (A only)
   TungOp top;       // Tungsten operator scalars
@@ -330,10 +330,13 @@ __device__ __forceinline__ void tile_store(const T *sr, const T *si, int nvalid,
   }
 }
 
-// ZM_PFC with a.keep set and ZM_KEEP are the z passes of a kept-spectrum run: the
-// combined spectrum stays in A (the next step's Psi, forward transforms
-// included) and its inverse goes to B.  ZM_KEEP takes A as such a spectrum, so
-// only N is transformed forward.
+// ZM_FIRST and ZM_KEEP are the z passes of a kept-spectrum run: the combined
+// spectrum stays in A (the next step's Psi, forward transforms included; a.keep:
+// not after the run's last step) and its inverse goes to B.  ZM_KEEP takes A as
+// such a spectrum, so only N is transformed forward.  ZM_FIRST is a mode of its
+// own: with the store behind a flag in ZM_PFC, single steps of 1024-point lines
+// took 395 us in this pass at 256x256x1024 FP64 (r16x16x4/E16/G2/split/mtp) and
+// take 295 without.
 // opL*h + opN*v of one mode; double-butterfly plans combine unrounded in double.
 template <typename Plan, typename T, typename M>
 __device__ __forceinline__ cplx<T> z_combine(cplx<T> h, cplx<T> v, M opl, M opn) {
@@ -408,11 +411,11 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
       multipliers();
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        if constexpr (MODE == ZM_PFC) acc[e] = ld_line<NT>(la + (t + TL * e));
+        if constexpr (MODE == ZM_PFC || MODE == ZM_FIRST) acc[e] = ld_line<NT>(la + (t + TL * e));
         v[e] = ld_line<NT>(lb + (t + TL * e));
       }
     }
-    if constexpr (MODE == ZM_PFC) {
+    if constexpr (MODE == ZM_PFC || MODE == ZM_FIRST) {
       // A = Fz^-1(opL*Fz(A) + opN*Fz(B))
       LineFft<T, Plan, -1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
       if constexpr (!Plan::XP) {
@@ -440,14 +443,13 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
       if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
     }
   }
-  if ((MODE == ZM_PFC || MODE == ZM_KEEP) && a.keep && active) {
+  if ((MODE == ZM_FIRST || (MODE == ZM_KEEP && a.keep)) && active) {
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<NT>(la + (t + TL * e), acc[e]);
   }
   LineFft<T, Plan, +1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
   if (active) {
-    cplx<T> *__restrict__ out =
-        (MODE == ZM_TMF || MODE == ZM_KEEP || (MODE == ZM_PFC && a.keep)) ? lb : la;
+    cplx<T> *__restrict__ out = MODE == ZM_PFC || MODE == ZM_TCOMB ? la : lb;
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<NT>(out + (t + TL * e), acc[e]);
   }
@@ -536,7 +538,7 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz_mt(TStepArgs<T> a) {
     }
 #pragma unroll
     for (int e = 0; e < E; ++e) acc[e] = c_scale(acc[e], (T)ta[slot(e)]);
-  } else if constexpr (MODE == ZM_PFC) {
+  } else if constexpr (MODE == ZM_PFC || MODE == ZM_FIRST) {
     // A = Fz^-1(opL*Fz(A) + opN*Fz(B))
     LineFft<T, Plan, -1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
     if constexpr (!Plan::XP) {
@@ -564,14 +566,13 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz_mt(TStepArgs<T> a) {
       acc[e] = z_combine<Plan>(acc[e], v[e], ta[slot(e)], tb[slot(e)]);
     if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
   }
-  if ((MODE == ZM_PFC || MODE == ZM_KEEP) && a.keep && active) {
+  if ((MODE == ZM_FIRST || (MODE == ZM_KEEP && a.keep)) && active) {
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<true>(la + (t + TL * e), acc[e]);
   }
   LineFft<T, Plan, +1, SPLIT, true, row_wave<Plan>()>::run(acc, t, ll, a.tw_z);
   if (active) {
-    cplx<T> *__restrict__ out =
-        (MODE == ZM_TMF || MODE == ZM_KEEP || (MODE == ZM_PFC && a.keep)) ? lb : la;
+    cplx<T> *__restrict__ out = MODE == ZM_PFC || MODE == ZM_TCOMB ? la : lb;
 #pragma unroll
     for (int e = 0; e < E; ++e) st_line<true>(out + (t + TL * e), acc[e]);
   }

@@ -377,6 +377,9 @@ hipError_t tz_launch(TStepArgs<T> a, hipStream_t s) {
   case ZM_KEEP:
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP>), grid, block, 0, s, a);
     break;
+  case ZM_FIRST:
+    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST>), grid, block, 0, s, a);
+    break;
   default:
     return hipErrorInvalidValue;
   }
@@ -445,6 +448,9 @@ hipError_t tz_pre_launch(TStepArgs<T> a, hipStream_t s) {
   case ZM_KEEP:
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP, true>), grid, block, 0, s, a);
     break;
+  case ZM_FIRST:
+    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST, true>), grid, block, 0, s, a);
+    break;
   default:
     return hipErrorInvalidValue;
   }
@@ -469,6 +475,9 @@ hipError_t tz_mt_launch(TStepArgs<T> a, hipStream_t s) {
     break;
   case ZM_KEEP:
     hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_KEEP, PAIR>), grid, block, 0, s, a);
+    break;
+  case ZM_FIRST:
+    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_FIRST, PAIR>), grid, block, 0, s, a);
     break;
   default:
     return hipErrorInvalidValue;
