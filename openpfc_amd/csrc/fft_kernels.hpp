@@ -562,7 +562,12 @@ __device__ __forceinline__ void z_mode_ops(const PfcOp &o, const TungOp &p,
 // holds one or two waves, so the evaluations are a serial chain no other wave
 // hides.  Above kZTabMax points the table (16 bytes a pair and column in
 // double) would take the LDS of the blocks that hide latency there, and the
-// pairs are evaluated per element.  Same values and arithmetic either way.
+// pairs are evaluated per element: before the transforms where two spectra are
+// loaded anyway, after the transform in ZM_TMF, which has one line in flight and
+// registers to lose (E multipliers held across its transform took 94 to 196
+// VGPRs at 512 points; us of the first variant with them before | after the
+// transform, FP32 192x96x1024 88.4 | 79.8, 96x96x512 27.9 | 25.5, 24x48x1024
+// 28.9 | 26.2).  Same values and arithmetic either way.
 // ----------------------------------------------------------------------------
 template <typename T> struct PfcZArgs {
   int zero_k0; // mean-split step: the k = 0 mode of the deviation stays 0
@@ -613,7 +618,7 @@ __global__ void __launch_bounds__(L *Plan::TL) k_pfc_z(PfcZArgs<T> a) {
   };
 
   cplx<T> acc[E], v[E];
-  T mul[TAB ? 1 : 2 * E];
+  T mul[TAB || MODE == ZM_TMF ? 1 : 2 * E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const long i = base + (long)(t + TL * e) * a.s_pos;
@@ -629,7 +634,7 @@ __global__ void __launch_bounds__(L *Plan::TL) k_pfc_z(PfcZArgs<T> a) {
       if constexpr (MODE != ZM_TMF) tab[NH * L + k * L + c] = (T)mb;
     }
     __syncthreads(); // the table is complete
-  } else {
+  } else if constexpr (MODE != ZM_TMF) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
       double ma, mb;
@@ -639,8 +644,15 @@ __global__ void __launch_bounds__(L *Plan::TL) k_pfc_z(PfcZArgs<T> a) {
     }
   }
   auto mul_a = [&](int e) {
-    if constexpr (TAB) return tab[slot(e)];
-    else return mul[e];
+    if constexpr (TAB) {
+      return tab[slot(e)];
+    } else if constexpr (MODE == ZM_TMF) {
+      double ma, mb;
+      z_mode_ops<MODE>(op, a.top, kxy, pfc_kc(t + TL * e, op.nz, op.fz), ma, mb);
+      return (T)ma;
+    } else {
+      return mul[e];
+    }
   };
   auto mul_b = [&](int e) {
     if constexpr (TAB) return tab[NH * L + slot(e)];
