@@ -412,7 +412,7 @@ hipError_t col_pass(pfc_hip_plan_s *p, int axis, int dir, const void *src0,
   a.src[1] = (const cplx<T> *)src1;
   a.dst[1] = (cplx<T> *)dst1;
   a.tw = twp<T>(p, n, v.plan_id);
-  a.W = p->W;
+  a.W = (short)p->W;
   a.s_pos = axis == 1 ? (long)pitch : (long)pitch * p->ny;
   a.s_outer = axis == 1 ? (long)pitch * p->ny : (long)pitch;
   // y columns of a batched plan run over the z planes of every field

@@ -114,9 +114,11 @@ template <typename T> int xcd_run_log2(long pitch, int partners) {
 template <typename T, typename Plan, int L, bool S>
 hipError_t col_launch(int dir, ColArgs<T> a, long n_outer, int nfields,
                       hipStream_t s) {
-  a.ntx = (a.W + L - 1) / L;
-  a.lg = xcd_run_log2<T>(a.s_pos | a.s_outer, (int)line_partners<T, L>());
-  dim3 grid((unsigned)(a.ntx * n_outer), (unsigned)nfields), block(L * Plan::TL);
+  a.ntx = (short)((a.W + L - 1) / L);
+  const unsigned blocks = (unsigned)(a.ntx * n_outer);
+  const int lg = xcd_run_log2<T>(a.s_pos | a.s_outer, (int)line_partners<T, L>());
+  a.runs = (blocks >> (lg + 3) << (lg + 3)) | (unsigned)lg;
+  dim3 grid(blocks, (unsigned)nfields), block(L * Plan::TL);
   if (dir < 0)
     hipLaunchKernelGGL((k_col<T, Plan, -1, L, S>), grid, block, 0, s, a);
   else
