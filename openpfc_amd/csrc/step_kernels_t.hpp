@@ -337,16 +337,6 @@ __device__ __forceinline__ void tile_store(const T *sr, const T *si, int nvalid,
 // own: with the store behind a flag in ZM_PFC, single steps of 1024-point lines
 // took 395 us in this pass at 256x256x1024 FP64 (r16x16x4/E16/G2/split/mtp) and
 // take 295 without.
-// opL*h + opN*v of one mode; double-butterfly plans combine unrounded in double.
-template <typename Plan, typename T, typename M>
-__device__ __forceinline__ cplx<T> z_combine(cplx<T> h, cplx<T> v, M opl, M opn) {
-  if constexpr (Plan::XP)
-    return cplx<T>{(T)((double)h.x * opl + (double)v.x * opn),
-                   (T)((double)h.y * opl + (double)v.y * opn)};
-  else
-    return c_add(c_scale(h, (T)opl), c_scale(v, (T)opn));
-}
-
 template <typename T, typename Plan, int G, bool SPLIT, int MODE, bool PRE = false,
           bool NT = false>
 __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
@@ -438,7 +428,7 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
 #pragma unroll
       for (int e = 0; e < E; ++e) {
         const cplx<T> h = PRE ? acc[e] : ld_line<NT>(la + (t + TL * e));
-        acc[e] = z_combine<Plan>(h, v[e], opl[e], opn[e]);
+        acc[e] = c_add(c_scale(h, opl[e]), c_scale(v[e], opn[e]));
       }
       if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
     }
@@ -563,7 +553,7 @@ __global__ void __launch_bounds__(G *Plan::TL) k_tz_mt(TStepArgs<T> a) {
     LineFft<T, Plan, -1, SPLIT, true, row_wave<Plan>()>::run(v, t, ll, a.tw_z);
 #pragma unroll
     for (int e = 0; e < E; ++e)
-      acc[e] = z_combine<Plan>(acc[e], v[e], ta[slot(e)], tb[slot(e)]);
+      acc[e] = c_add(c_scale(acc[e], ta[slot(e)]), c_scale(v[e], tb[slot(e)]));
     if (MODE == ZM_KEEP && a.zero_k0 && l == 0 && t == 0) acc[0] = cplx<T>{0, 0};
   }
   if ((MODE == ZM_FIRST || (MODE == ZM_KEEP && a.keep)) && active) {

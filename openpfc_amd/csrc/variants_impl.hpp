@@ -366,24 +366,29 @@ template <typename T, typename Plan, int G, bool S, bool TILE>
 hipError_t tz_launch(TStepArgs<T> a, hipStream_t s) {
   const long lines = (long)a.W * a.ny;
   dim3 grid((unsigned)((lines + G - 1) / G)), block(G * Plan::TL);
-  switch (a.mode) {
-  case ZM_PFC:
+  if constexpr (Plan::XP) { // plans of the PFC model's single steps
+    if (a.mode != ZM_PFC) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_PFC>), grid, block, 0, s, a);
-    break;
-  case ZM_TMF:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TMF>), grid, block, 0, s, a);
-    break;
-  case ZM_TCOMB:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB>), grid, block, 0, s, a);
-    break;
-  case ZM_KEEP:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP>), grid, block, 0, s, a);
-    break;
-  case ZM_FIRST:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST>), grid, block, 0, s, a);
-    break;
-  default:
-    return hipErrorInvalidValue;
+  } else {
+    switch (a.mode) {
+    case ZM_PFC:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_PFC>), grid, block, 0, s, a);
+      break;
+    case ZM_TMF:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TMF>), grid, block, 0, s, a);
+      break;
+    case ZM_TCOMB:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB>), grid, block, 0, s, a);
+      break;
+    case ZM_KEEP:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP>), grid, block, 0, s, a);
+      break;
+    case ZM_FIRST:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST>), grid, block, 0, s, a);
+      break;
+    default:
+      return hipErrorInvalidValue;
+    }
   }
   return hipGetLastError();
 }
@@ -437,24 +442,29 @@ template <typename T, typename Plan, int G, bool S>
 hipError_t tz_pre_launch(TStepArgs<T> a, hipStream_t s) {
   const long lines = (long)a.W * a.ny;
   dim3 grid((unsigned)((lines + G - 1) / G)), block(G * Plan::TL);
-  switch (a.mode) {
-  case ZM_PFC:
+  if constexpr (Plan::XP) { // plans of the PFC model's single steps
+    if (a.mode != ZM_PFC) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_PFC, true>), grid, block, 0, s, a);
-    break;
-  case ZM_TMF:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TMF, true>), grid, block, 0, s, a);
-    break;
-  case ZM_TCOMB:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB, true>), grid, block, 0, s, a);
-    break;
-  case ZM_KEEP:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP, true>), grid, block, 0, s, a);
-    break;
-  case ZM_FIRST:
-    hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST, true>), grid, block, 0, s, a);
-    break;
-  default:
-    return hipErrorInvalidValue;
+  } else {
+    switch (a.mode) {
+    case ZM_PFC:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_PFC, true>), grid, block, 0, s, a);
+      break;
+    case ZM_TMF:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TMF, true>), grid, block, 0, s, a);
+      break;
+    case ZM_TCOMB:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_TCOMB, true>), grid, block, 0, s, a);
+      break;
+    case ZM_KEEP:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_KEEP, true>), grid, block, 0, s, a);
+      break;
+    case ZM_FIRST:
+      hipLaunchKernelGGL((k_tz<T, Plan, G, S, ZM_FIRST, true>), grid, block, 0, s, a);
+      break;
+    default:
+      return hipErrorInvalidValue;
+    }
   }
   return hipGetLastError();
 }
@@ -465,24 +475,29 @@ hipError_t tz_mt_launch(TStepArgs<T> a, hipStream_t s) {
   const long lines = (long)a.W * a.ny;
   const long blocks = PAIR ? (long)a.W * ((a.ny + 1) / 2) : (lines + G - 1) / G;
   dim3 grid((unsigned)blocks), block(G * Plan::TL);
-  switch (a.mode) {
-  case ZM_PFC:
+  if constexpr (Plan::XP) { // plans of the PFC model's single steps
+    if (a.mode != ZM_PFC) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_PFC, PAIR>), grid, block, 0, s, a);
-    break;
-  case ZM_TMF:
-    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_TMF, PAIR>), grid, block, 0, s, a);
-    break;
-  case ZM_TCOMB:
-    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_TCOMB, PAIR>), grid, block, 0, s, a);
-    break;
-  case ZM_KEEP:
-    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_KEEP, PAIR>), grid, block, 0, s, a);
-    break;
-  case ZM_FIRST:
-    hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_FIRST, PAIR>), grid, block, 0, s, a);
-    break;
-  default:
-    return hipErrorInvalidValue;
+  } else {
+    switch (a.mode) {
+    case ZM_PFC:
+      hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_PFC, PAIR>), grid, block, 0, s, a);
+      break;
+    case ZM_TMF:
+      hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_TMF, PAIR>), grid, block, 0, s, a);
+      break;
+    case ZM_TCOMB:
+      hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_TCOMB, PAIR>), grid, block, 0, s, a);
+      break;
+    case ZM_KEEP:
+      hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_KEEP, PAIR>), grid, block, 0, s, a);
+      break;
+    case ZM_FIRST:
+      hipLaunchKernelGGL((k_tz_mt<T, Plan, G, S, ZM_FIRST, PAIR>), grid, block, 0, s, a);
+      break;
+    default:
+      return hipErrorInvalidValue;
+    }
   }
   return hipGetLastError();
 }
