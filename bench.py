@@ -13,11 +13,11 @@ psi_hat = opL*F(psi) + opN*F(psi^3), psi = F^-1(psi_hat)
     python bench.py --model tungsten     # Tungsten mean-field step (see below)
 
 Prints one JSON line.  `value` is FP64 steps/s with the field resident in
-HBM, timed over one K-step call (which fuses step boundaries when the
-autotuner found that faster); `step_hbm_frac` is the per-step model bytes
-2R + 12C (R a real field, C a half spectrum) over the step time, and
-`run_hbm_frac` the bytes the timed run itself needs per step (12C + 2R/K when
-step boundaries are fused).  The same workload in FP32-mixed mode (FP32 deviation field and
+HBM, timed over one K-step call (which keeps psi's spectrum between steps when
+the autotuner found that faster); `run_bytes_per_step` is what that call has to
+move per step (R a real field, C a half spectrum: 10C and, per run of steps on
+one spectrum, 2C + 2R; 12C + 2R for single steps), and `step_hbm_frac` and
+`run_hbm_frac` are those bytes over the step time.  The same workload in FP32-mixed mode (FP32 deviation field and
 transforms, FP64 conserved mean) is reported under "fp32_mixed" with its
 error against the FP64 run after the same steps.  `roofline` is the
 dominant kernel's algorithmic bytes per launch over its mean launch duration
@@ -168,6 +168,27 @@ def fused_pass_bytes(n: int, esize: int):
     N: y forward 2C, z 2C + 2C, y inverse 2C, boundary C + C."""
     C = 2 * esize * (n // 2 + 1) * n * n
     return {"y_fwd": 2 * C, "z_fused": 4 * C, "y_inv": 2 * C, "x_boundary_fused": 2 * C}
+
+
+def kept_run_steps(eps: float, dt: float) -> int:
+    """Most steps the library takes on one kept spectrum (8 over the largest
+    growth exponent of a mode, at most 64)."""
+    if not dt > 0:
+        return 1
+    top = 1.0 + math.sqrt(max(-eps, 0.0))
+    g = max(-k2 * (eps + (1.0 - k2) ** 2) * dt
+            for k2 in (top * i / 512 for i in range(1, 513)))
+    return 64 if g * 64 <= 8.0 else max(1, int(8.0 / g))
+
+
+def run_step_bytes(n: int, esize: int, steps: int, span: int) -> float:
+    """Algorithmic bytes per step of a call of `steps` steps that keeps the
+    spectrum over runs of at most `span`.  A run of k steps moves 10kC + 2C + 2R:
+    12C + R for the first step but its inverse x, 10C for each following one, less
+    the C the last z pass does not keep, and C + R of the inverse x."""
+    R = esize * n ** 3
+    C = 2 * esize * (n // 2 + 1) * n * n
+    return 10 * C + -(-steps // span) * (2 * C + 2 * R) / steps
 
 
 def tung_pass_bytes(n: int, esize: int):
@@ -867,8 +888,8 @@ def main(argv=None):
     layout = chosen64.get("step_layout", "natural")
     fused = kf[5] > 0
     if fused:
-        # the timed K-step call fuses step boundaries: its steady-state
-        # passes are y forward, z, y inverse and the fused boundary
+        # the timed K-step call keeps psi's spectrum: its steady-state
+        # passes are y forward, z, y inverse and the step boundary
         fb = fused_pass_bytes(n, 8)
         fk = dict(zip(FUSED_NAMES, kf))
         dname = max(fb, key=lambda k: fk[k])
@@ -877,7 +898,7 @@ def main(argv=None):
                       "y_inv": ("k_ty_inv", "t_y_inv"),
                       "x_boundary_fused": ("k_tx_bnd", "t_x_fuse")}[dname]
         alg_launch = fb[dname]
-        run_bytes = sum(fb.values()) + 2 * 8 * n ** 3 / args.steps
+        run_bytes = run_step_bytes(n, 8, args.steps, kept_run_steps(r, dt))
     else:
         dom = max(range(5), key=lambda i: kms[i])
         dname = PASS_NAMES[dom]
@@ -912,8 +933,8 @@ def main(argv=None):
                    "dx": dx, "dt": dt, "r": r, "psi_mean": -0.2, "noise": 0.01,
                    "seed_radius": 64 * dx, "seed_amplitude": SEED_AMP},
         "ns_per_dof_step": ms64 * 1e6 / n ** 3,
-        "step_hbm_frac": step_bytes / (ms64 * 1e-3) / HBM_PEAK,
-        "step_alg_bytes": step_bytes,
+        "step_hbm_frac": run_bytes / (ms64 * 1e-3) / HBM_PEAK,
+        "step_alg_bytes": run_bytes,
         "run_bytes_per_step": run_bytes,
         "run_hbm_frac": run_bytes / (ms64 * 1e-3) / HBM_PEAK,
         "wall_s_timed": wall64,
@@ -962,16 +983,15 @@ def main(argv=None):
             del d, got, diff, st, fft
             torch.cuda.empty_cache()
             log(f"{key}: {ms32:.3f} ms/step")
+            bytes32 = (run_step_bytes(n, 4, args.steps, kept_run_steps(r, dt))
+                       if k32f[5] > 0 else sum(pass_bytes(n, 4).values()))
             out[key] = {
                 "mode": mode,
                 "steps_per_s": 1000.0 / ms32, "ms_per_step": ms32,
                 "ns_per_dof_step": ms32 * 1e6 / n ** 3,
                 "speedup_vs_fp64": ms64 / ms32,
-                "step_hbm_frac": sum(pass_bytes(n, 4).values()) / (ms32 * 1e-3) / HBM_PEAK,
-                "run_hbm_frac": ((sum(fused_pass_bytes(n, 4).values())
-                                  + 2 * 4 * n ** 3 / args.steps)
-                                 if k32f[5] > 0 else sum(pass_bytes(n, 4).values()))
-                                / (ms32 * 1e-3) / HBM_PEAK,
+                "step_hbm_frac": bytes32 / (ms32 * 1e-3) / HBM_PEAK,
+                "run_hbm_frac": bytes32 / (ms32 * 1e-3) / HBM_PEAK,
                 "kernels_ms": dict(zip(PASS_NAMES, k32)),
                 "fused_run_ms": dict(zip(FUSED_NAMES, k32f)) if k32f[5] > 0 else None,
                 "variants": chosen32,
@@ -991,7 +1011,7 @@ def main(argv=None):
     sc = stream_copy(P, torch, 16 * (n // 2 + 1) * n * n)
     out["stream_copy"] = sc
     out["roofline"]["frac_of_stream_copy"] = out["roofline"]["achieved"] / sc["GBps"]
-    out["step_frac_of_stream_copy"] = step_bytes / (ms64 * 1e-3) / 1e9 / sc["GBps"]
+    out["step_frac_of_stream_copy"] = run_bytes / (ms64 * 1e-3) / 1e9 / sc["GBps"]
 
     # ---- the C++ drop-in path (App over PFCModelHIP), same variants -------
     if not args.no_cpp:
