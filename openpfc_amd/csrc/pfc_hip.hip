@@ -232,9 +232,8 @@ int upload_line_tables(pfc_hip_plan_s *p, int n) {
   for (int pid = 0; pid < plan_count(n); ++pid) {
     auto key = std::make_pair(n, pid);
     if (p->tw.count(key)) continue;
-    void *d = nullptr;
-    if (int rc = upload_table(p, &d, line_twiddles(n, pid), "line twiddles")) return rc;
-    p->tw[key] = d;
+    // into the plan's slot, which is freed with the plan if the upload fails
+    if (int rc = upload_table(p, &p->tw[key], line_twiddles(n, pid), "line twiddles")) return rc;
   }
   return 0;
 }
@@ -255,9 +254,8 @@ int upload_plane_tables(pfc_hip_plan_s *p) {
   for (int row = 0; row < 2; ++row) {
     const int n = row ? p->nx / 2 : p->ny;
     const int pid = p->prec == PFC_HIP_F64 ? plane_pid<double>(row) : plane_pid<float>(row);
-    void *d = nullptr;
-    if (int rc = upload_table(p, &d, line_twiddles(n, pid), "plane twiddles")) return rc;
-    p->tw[std::make_pair(n, pid)] = d;
+    if (int rc = upload_table(p, &p->tw[{n, pid}], line_twiddles(n, pid), "plane twiddles"))
+      return rc;
   }
   return p->prec == PFC_HIP_F64 ? 0 : upload_wn64(p);
 }
