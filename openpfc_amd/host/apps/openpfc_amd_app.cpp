@@ -4,7 +4,7 @@
 //
 // model.name selects the model: "tungsten" (TungstenHIP<double>; with
 // plan_options.precision "float", TungstenHIP<float>) or "pfc"
-// (PFCModelHIP, params {epsilon}).  Mirrors the reference's tungsten
+// (PFCModelHIP, params {epsilon, optional keep_spectrum}).  Mirrors the reference's tungsten
 // application entry (apps/tungsten/include/tungsten/common/
 // tungsten_app_main.hpp): errors are printed and the exit status is 1.
 #include <openpfc_amd/app.hpp>

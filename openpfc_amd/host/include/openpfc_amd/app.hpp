@@ -267,7 +267,15 @@ template <> struct ModelTraits<PFCModelHIP> {
   static constexpr int precision = PFC_HIP_F64;
   static const char *name() { return "pfc"; }
   static std::unique_ptr<PFCModelHIP> create(fft::HipFft &f, const World &w, const Value &p) {
-    return std::make_unique<PFCModelHIP>(f, w, num(p, "epsilon", "model.params (pfc)"));
+    auto m = std::make_unique<PFCModelHIP>(f, w, num(p, "epsilon", "model.params (pfc)"));
+    // false: a run does not depend on its save interval in the last digits
+    if (const Value *k = p.find("keep_spectrum")) {
+      if (!k->is_bool())
+        throw std::invalid_argument("model.params (pfc): 'keep_spectrum' must be true or false, got " +
+                                    k->dump());
+      m->set_keep_spectrum(k->as_bool());
+    }
+    return m;
   }
 };
 

@@ -40,7 +40,18 @@ public:
     // step variants from the autotune cache, or tuned now (autotune.hpp)
     m_tuned = gpu::tune_step(m_hfft.plan(), m_psi.data(),
                              gpu::step_key("pfc", PFC_HIP_F64, w.size, false), m_hfft.stream());
+    if (!m_keep_spectrum)
+      pfc::detail::check_abi(pfc_hip_variant_set(m_hfft.plan(), PFC_HIP_ROLE_STEP_FUSE, 0),
+                             "PFCModelHIP::initialize");
   }
+
+  // Whether multi-step calls may keep psi's spectrum between their steps (the
+  // default; faster).  Such a call agrees with its single steps to rounding, so
+  // that a trajectory depends in its last digits on where step_n calls, and with
+  // them the save points, cut it; false makes every call the bits of its single
+  // steps.  Takes effect at initialize().
+  void set_keep_spectrum(bool on) noexcept { m_keep_spectrum = on; }
+  bool get_keep_spectrum() const noexcept { return m_keep_spectrum; }
 
   // How initialize() chose the step's launch variants.
   gpu::TuneOutcome autotune_outcome() const noexcept { return m_tuned; }
@@ -105,6 +116,7 @@ private:
   RealField m_density;
   core::DataBuffer<backend::HipTag, double> m_psi;
   bool m_host_stale = false;
+  bool m_keep_spectrum = true;
   gpu::TuneOutcome m_tuned = gpu::TuneOutcome::defaults;
 };
 

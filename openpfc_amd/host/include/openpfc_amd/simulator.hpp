@@ -59,8 +59,9 @@ public:
   // Up to max_steps steps with the effect of that many step() calls (no
   // reference counterpart: the reference loops over step()).  Without
   // boundary conditions nothing happens between two steps up to the next
-  // save point, so those steps go to Model::step_many in one call; returns
-  // the number of steps taken.
+  // save point, so those steps go to Model::step_many in one call (equal to
+  // single steps to rounding where the model keeps its spectrum between them:
+  // PFCModelHIP::set_keep_spectrum); returns the number of steps taken.
   int step_block(int max_steps) {
     if (max_steps <= 1 || m_time.get_increment() == 0 || !m_bcs.empty()) {
       step();
