@@ -14,7 +14,9 @@
 //                                    "."), named <device>_autotune_cache.json.
 // An entry is keyed by model, precision, extents and the mean-split mode and
 // holds the variant name chosen for every step role; an entry naming a
-// variant the library no longer offers counts as missing.  What is tuned
+// variant the library no longer offers counts as missing, except that
+// cache_only, which cannot tune, takes an entry of an earlier build and leaves
+// the roles whose named variants were since removed at their defaults.  What is tuned
 // here is the library's launch shape per pass (radix plan, lines per block,
 // layout), where the reference tunes block sizes of its elementwise kernels.
 #pragma once
@@ -60,9 +62,18 @@ inline std::string step_key(const std::string &model, int precision, const Int3 
          (mean_split ? "/mean_split" : "");
 }
 
+// Names that earlier builds stored and that no plan offers any more: step
+// boundaries that paired an nx/2- with an nx-point plan (role 15, "A+B/..."), and
+// z passes with non-temporal lines but no multiplier table (role 9, ".../nt").
+inline bool removed_variant(int role, const std::string &name) {
+  if (role == PFC_HIP_ROLE_T_X_FUSE) return name.find('+') != std::string::npos;
+  return role == PFC_HIP_ROLE_T_Z && name.size() > 3 && name.ends_with("/nt");
+}
+
 // Select the variants of a cached entry; false (nothing changed) when any
-// role's name is not offered by the plan.
-inline bool apply_entry(pfc_hip_plan_t plan, const json::Value &entry) {
+// role's name is not offered by the plan.  With skip_removed, roles with a
+// removed_variant keep what they are at.
+inline bool apply_entry(pfc_hip_plan_t plan, const json::Value &entry, bool skip_removed = false) {
   if (!entry.is_object()) return false;
   std::vector<std::pair<int, int>> picks;
   for (int role = 0; role < 64; ++role) {
@@ -76,6 +87,8 @@ inline bool apply_entry(pfc_hip_plan_t plan, const json::Value &entry) {
       const char *nm = pfc_hip_variant_name(plan, role, i);
       if (nm && v->is_string() && v->as_string() == nm) found = i;
     }
+    if (found < 0 && skip_removed && v->is_string() && removed_variant(role, v->as_string()))
+      continue;
     if (found < 0) return false;
     picks.emplace_back(role, found);
   }
@@ -139,7 +152,7 @@ inline TuneOutcome tune_step(pfc_hip_plan_t plan, void *psi, const std::string &
   json::Value cache = load_cache(path);
   if (const json::Value *entries = cache.find("entries"))
     if (const json::Value *e = entries->find(key))
-      if (apply_entry(plan, *e)) return TuneOutcome::cached;
+      if (apply_entry(plan, *e, mode == "cache_only")) return TuneOutcome::cached;
   if (mode == "cache_only")
     throw std::runtime_error("No cached configuration for kernel: " + key + " (" + path + ")");
   pfc::detail::check_abi(pfc_hip_pfc_autotune(plan, psi, 3, stream, nullptr, 0),
