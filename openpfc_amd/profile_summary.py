@@ -16,7 +16,9 @@ counter reads for the plain device-to-device copy of `bench.py
 --calibrate-copy`, which reads and writes 4 GiB per dispatch and runs last:
 the calibration value is the median over the trailing __amd_rocclr_copyBuffer
 dispatches with the grid size of the last one (other copies, such as the
-autotuner's backup of the field, come earlier and differ in size).  The scaled bytes per dispatch of every kernel go to the
+autotuner's backup of the field, come earlier and differ in size).  The scaled
+bytes of every kernel's median dispatch (a run's last z pass keeps no spectrum
+and moves less than the others) go to the
 markdown table and, for the FP64 kernels, with --traffic-json to a JSON file
 ({name: [GB read, GB written]}) bench.py uses for roofline.traffic.
 """
@@ -28,6 +30,7 @@ import glob
 import json
 import os
 import re
+import statistics
 from collections import defaultdict
 
 COPY_BYTES = 4 << 30  # bench.py --calibrate-copy: 4 GiB read + 4 GiB written
@@ -75,7 +78,7 @@ def kernel_stats(trace_dir: str):
     return out
 
 
-def counter_means(pmc_dir: str):
+def counter_medians(pmc_dir: str):
     rows = _csv(pmc_dir, "counter_collection.csv")
     per = defaultdict(list)
     copy = []
@@ -95,7 +98,7 @@ def counter_means(pmc_dir: str):
             tail.append(v)
         tail.sort()
         cal = tail[len(tail) // 2]
-    return {k: sum(v) / len(v) for k, v in per.items()}, cal
+    return {k: statistics.median(v) for k, v in per.items()}, cal
 
 
 def busy_window(trace_dir: str, gap_ms: float):
@@ -249,8 +252,8 @@ def main(argv=None):
                          f"{(w['span_ms'] - w['busy_ms']) / a.window_steps:.4f} ms idle.")
     traffic = {}
     if a.fetch and a.write:
-        fm, fcopy = counter_means(a.fetch)
-        wm, wcopy = counter_means(a.write)
+        fm, fcopy = counter_medians(a.fetch)
+        wm, wcopy = counter_medians(a.write)
         if not fcopy or not wcopy:
             raise RuntimeError("no copy-kernel dispatch in the PMC runs (use --calibrate-copy)")
         sf = COPY_BYTES / (fcopy * 1024.0)
