@@ -40,8 +40,8 @@ __device__ __forceinline__ void pfc_op_deriv(const PfcOp &o, double kxy, double 
 // kz enters as kz*kz only, so up to kZTabMax points the four multipliers of a
 // column come from an LDS table of nz/2 + 1 entries (see k_pfc_z); beyond that
 // they are evaluated per element.  Bound by memory and by the latency of the four
-// or five dependent line transforms: at 128^3 FP64 33.0 us (5 spectra of 17 MB,
-// 2.6 TB/s) against 3*16.3 + 15.5 + 2*11.0 = 86.4 us of the separate passes.
+// or five dependent line transforms: at 128^3 FP64 27.2 us (5 spectra of 17 MB,
+// 3.1 TB/s) against 3*16.3 + 15.5 + 2*11.0 = 86.4 us of the separate passes.
 struct AdjZArgs {
   const cplx<double> *lam;
   cplx<double> *P, *N;

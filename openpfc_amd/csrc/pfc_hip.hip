@@ -256,7 +256,7 @@ int upload_wn64(pfc_hip_plan_s *p) {
 // the same radices has them already, and in single precision the real-FFT twiddles
 // in double.  One copy in all, as without the plane kernels: with one for each table
 // a 32^3 FP64 stepper took 427 us to make against 339, and an ensemble of seven plans
-// 3.05 ms against 2.56 (now under 370 us, and 2.82 ms with its buffers C).
+// 3.05 ms against 2.56 (now within 10 %, and 2.82 ms with its buffers C).
 int upload_real_tables(pfc_hip_plan_s *p, bool plane) {
   const bool f64 = p->prec == PFC_HIP_F64;
   std::vector<unsigned char> bytes;
@@ -793,8 +793,9 @@ int step_transposed(pfc_hip_plan_s *p, void *psi, hipStream_t s, hipEvent_t *ev)
 //
 // Measured, ms per step of a run, tuned variants, kept spectrum against psi
 // transformed anew at a fused boundary (12C) and against single steps (12C + 2R):
-//   FP64 1024^3 17.6 / 21.1 / 23.1 (y 3.14, z 5.35, inverse y 3.47, boundary 4.09)
-//   FP32 1024^3  9.3 / 11.6 / 12.0 (y 1.60, z 2.76, inverse y 1.75, boundary 2.40)
+//   FP64 1024^3 17.2 / 21.1 / 23.1 (y 3.14, z 5.3 to 6.1 by where its two spectra
+//               land in memory, 4.2 in a run's last step, inverse y 3.46, boundary 4.11)
+//   FP32 1024^3  9.0 / 11.6 / 12.0 (y 1.60, z 3.03, inverse y 1.75, boundary 2.44)
 //   FP64  512^3 2.00 / 2.50 / 2.75,  FP32 512^3 1.07 / 1.34 / 1.42
 //   FP64  256^3 .245 / .334 / .363,  FP32 256^3 .134 / .156 / .188
 int fused_span(const PfcOp &o) {
@@ -1107,8 +1108,8 @@ int sum_partials(double *part, int n, double *out, hipStream_t s) {
 // Adjoint of one plain PFC step, double fields, with the z transforms and the
 // spectral part in one pass (k_adj_z): x and y passes of psi, N(psi) and lambda
 // (one plane launch where the plane kernels are on), k_adj_z, inverse y and x with
-// the combine (one plane launch).  128^3 FP64: 33 + 33 + 31 us and the reduction's 6,
-// against 13 launches of 187 us pass by pass; 20 steps forward and back 4.24 ms
+// the combine (one plane launch).  128^3 FP64: 32 + 27 + 31 us and the reduction's 6,
+// against 13 launches of 187 us pass by pass; 20 steps forward and back 4.28 ms
 // (6.33 before).
 int adjoint_f64(pfc_hip_plan_s *p, const void *psi, void *lambda, double *dr, hipStream_t s) {
   using T = double;

@@ -334,9 +334,9 @@ __device__ __forceinline__ void tile_store(const T *sr, const T *si, int nvalid,
 // spectrum stays in A (the next step's Psi, forward transforms included; a.keep:
 // not after the run's last step) and its inverse goes to B.  ZM_KEEP takes A as
 // such a spectrum, so only N is transformed forward.  ZM_FIRST is a mode of its
-// own: with the store behind a flag in ZM_PFC, single steps of 1024-point lines
-// took 395 us in this pass at 256x256x1024 FP64 (r16x16x4/E16/G2/split/mtp) and
-// take 295 without.
+// own: the store costs registers (r16x16x4/E16/G2/split/mtp in double: 254 -> 282,
+// one wave a SIMD), and behind a flag in ZM_PFC it cost single steps as much (that
+// variant at 256x256x1024: 395 us against 295 without).
 template <typename T, typename Plan, int G, bool SPLIT, int MODE, bool PRE = false,
           bool NT = false>
 __global__ void __launch_bounds__(G *Plan::TL) k_tz(TStepArgs<T> a) {
