@@ -1259,25 +1259,34 @@ __global__ void __launch_bounds__(256) k_stream_copy(const uint4 *__restrict__ s
   if (i < n) dst[i] = src[i];
 }
 
-// Whether the plane kernels are the default of the x roles.  One block takes a
-// plane, so they need planes enough to keep the CUs busy and lose where few
-// large ones leave most of the chip idle.  Measured (us, plane against row and
-// column kernels; run = step of a multi-step run, one = single step):
-//   FP64 32x32x32    run 11.6 / 19.0  one 17.0 / 23.2  r2c 15.0 / 17.1
-//   FP64 64x64x64    run 15.9 / 23.6  one 20.4 / 24.1  r2c 14.4 / 16.6
-//   FP64 128x128x128 run 43.0 / 60.6  one 50.0 / 59.5  r2c 32.3 / 42.7
-//   FP32 96x96x96    run 26.6 / 36.1  one 32.2 / 36.4  r2c 17.6 / 21.5
-//   FP32 96x96x512   run 66.5 / 85.5  one 73.1 / 85.7  r2c 36.5 / 50.0
-//   FP32 256x64x64   run 25.4 / 33.7  one 33.8 / 33.2  r2c 19.5 / 21.0
-//   FP32 192x96x48   run 29.4 / 35.6  one 37.9 / 35.7  r2c 21.0 / 22.4
-//   FP64 128x128x32  run 31.1 / 32.5  one 38.6 / 32.1  r2c 21.3 / 19.3
-//   FP64 192x48x24   run 22.8 / 27.0  one 28.5 / 27.3  r2c 16.1 / 18.1
-// so: from 64 planes on, or where a plane's bytes are at most 1600 per plane
-// there is.  Above 140 KB (FP32 192x192: 149 KB) a CU holds one block and the
-// column passes are as fast (run 96.8 / 96.0, one 103 / 94.6 us at 192^3).
+// Whether the plane kernels are the default of the x roles: where no ordinary call
+// is slower than with the row and column kernels.  One block takes a plane, so they
+// need planes enough to keep the CUs busy.  Swept over 2127 extents of up to 2^23
+// points (us, plane / row and column kernels; run = step of a multi-step run, one =
+// single step):
+//   FP64 64x64x64    run 16.0 / 23.5  one 19.4 / 23.7  r2c 14.5 / 17.6  c2r 14.2 / 17.6
+//   FP64 128x128x96  run 41.4 / 52.4  one 47.4 / 53.1  r2c 25.4 / 30.1  c2r 24.8 / 28.2
+//   FP64 128x128x64  run 36.3 / 44.0  one 41.0 / 44.6  r2c 22.1 / 22.5  c2r 20.9 / 21.5
+//   FP64 128x128x32  run 30.6 / 32.9  one 37.1 / 33.5  r2c 19.1 / 18.0  c2r 18.0 / 17.3
+//   FP32 96x96x256   run 39.8 / 50.2  one 43.0 / 50.8  r2c 20.7 / 28.1  c2r 19.6 / 26.6
+//   FP32 128x128x128 run 35.8 / 45.6  one 40.4 / 46.1  r2c 20.8 / 23.0  c2r 19.9 / 22.1
+//   FP32 128x128x48  run 25.0 / 29.3  one 32.5 / 29.8  r2c 16.4 / 17.7  c2r 15.8 / 17.9
+//   FP32 512x32x48   run 26.9 / 29.1  one 34.0 / 29.8  r2c 19.2 / 17.7  c2r 16.3 / 17.6
+//   FP32 128x192x192 run 67.3 / 68.2  one 74.9 / 69.0  r2c 32.0 / 34.8  c2r 31.3 / 32.1
+//   FP32 64x512x128  run 93.9 / 69.3  one 110  / 70.1  r2c 40.9 / 36.2  c2r 41.5 / 33.4
+// so, in FP64 and up to 32 KB a plane: from 64 planes on, or where a plane's bytes
+// are at most 1600 per plane there is.  Larger FP32 planes against the faster FP32 row
+// kernels: at most 1000 up to 80 KB; above that a CU holds one block, so at most 800
+// and whole rounds of the 256 CUs (two blocks a plane).  Columns of 512 points run
+// one line a wave, in 8- or 16-byte pieces: never.  Above 140 KB the column passes
+// are as fast.  Over the extents this takes, single steps gain 1.22 (FP32) and 1.29
+// (FP64) times and runs 1.38 and 1.46; five of 1641 lose more than 3 % in some call, 6 %
+// at worst (with 64 planes or 1600 bytes for all: 72, and 36 %).
 bool plane_variant_default(const pfc_hip_plan_s *p) {
-  const size_t b = p->plane_bytes();
-  return b > 0 && b <= 140 * 1024 && (p->nz >= 64 || b <= (size_t)1600 * p->nz);
+  const size_t b = p->plane_bytes(), nz = (size_t)p->nz;
+  if (b == 0 || b > 140 * 1024 || p->ny >= 512) return false;
+  if (p->prec == PFC_HIP_F64 || b <= 32 * 1024) return nz >= 64 || b <= 1600 * nz;
+  return b <= 80 * 1024 ? b <= 1000 * nz : b <= 800 * nz && nz % 128 == 0;
 }
 
 // Default variants by line length, where another variant than the first of a
