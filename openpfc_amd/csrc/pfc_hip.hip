@@ -1378,11 +1378,10 @@ constexpr DefaultVariant kDefaultXp[] = {
     {ROLE_T_X_FWD, 256, "r16x16/E16/xp/G16/full/wide"},         // first 1.11, 1.15
     {ROLE_T_X_FWD, 512, "r8x8x8/E8/xp/G16/split/wide/nt"},      // 1.02
     {ROLE_T_X_FWD, 1024, "r16x16x4/E16/xp/G8/split/wide"},      // 1.13
-    {ROLE_T_Y_FWD, 128, "r16x8/E16/xp/G16/split/wide1"},        // 1.07
     {ROLE_T_Y_FWD, 256, "r16x16/E16/xp/G16/split/wide2/nt"},    // 1.11
     {ROLE_T_Y_FWD, 512, "r8x8x8/E8/xp/G16/split/wide2/nt"},     // 1.00, 1.12
     {ROLE_T_Y_FWD, 1024, "r16x16x4/E16/xp/G16/split/wide2/nt"}, // (as 256)
-    {ROLE_T_Z, 128, "r8x4x4/E8/xp/G4/full/mt"},                 // 1.06
+    {ROLE_T_Z, 128, "r8x4x4/E8/xp/G4/split/mt"},                // 1.01 to 1.04
     {ROLE_T_Z, 256, "r16x16/E16/xp/G4/split/mt"},               // 1.31
     {ROLE_T_Z, 512, "r8x8x8/E8/xp/G1/full/mt"},                 // 1.13
     {ROLE_T_Z, 1024, "r16x16x4/E16/xp/G2/split/mtp"},           // 1.2
@@ -1390,58 +1389,107 @@ constexpr DefaultVariant kDefaultXp[] = {
     {ROLE_T_Y_INV, 256, "r16x16/E16/xp/G16/split/wide2/nt"},    // 1.08 (in a run)
     {ROLE_T_Y_INV, 512, "r16x16x2/E16/xp/G16/split/wide2"},     // 1.00, 1.06
     {ROLE_T_Y_INV, 1024, "r16x16x4/E16/xp/G16/split/wide2"},
-    {ROLE_T_X_INV, 128, "r16x8/E16/xp/G16"},                    // 1.09 (in a run)
+    {ROLE_T_X_INV, 128, "r8x4x4/E8/xp/G16"},                    // 1.03 to 1.15
     {ROLE_T_X_INV, 256, "r16x16/E16/xp/G16"}};                  // 1.05
-// z pass of PFC plans whose three run spectra fit the last-level cache
-constexpr DefaultVariant kCachedZF64[] = {{ROLE_T_Z, 128, "r8x4x4/E8/G4/full"},
-                                          {ROLE_T_Z, 256, "r16x16/E16/G4/split"},
-                                          {ROLE_T_Z, 512, "r8x8x8/E8/G1/split/pre"}};
-constexpr DefaultVariant kCachedZF32[] = {{ROLE_T_Z, 128, "r16x8/E16/G8/full"},
-                                          {ROLE_T_Z, 256, "r8x8x4/E8/G2/full"},
-                                          {ROLE_T_Z, 512, "r8x8x8/E8/G2/split"}};
+// Transposed passes of PFC plans whose grids the 256 MB last-level cache holds: so
+// many spectra of the plan have to fit.
+struct CachedVariant {
+  DefaultVariant d;
+  int spectra;
+};
+constexpr size_t kLastLevelCache = 256u << 20;
+constexpr CachedVariant kCachedF64[] = {
+    {{ROLE_T_X_FWD, 256, "r4x4x4x4/E4/G8/split/wide"}, 3},
+    {{ROLE_T_X_FWD, 512, "r8x8x8/E8/G8/full/wide"}, 3},
+    {{ROLE_T_Y_FWD, 128, "r8x4x4/E8/G8/split/wide4"}, 3},
+    {{ROLE_T_Y_FWD, 256, "r16x16/E16/G8/split/wide4"}, 3},
+    {{ROLE_T_Z, 128, "r8x4x4/E8/G4/full"}, 3},
+    {{ROLE_T_Z, 256, "r16x16/E16/G4/split"}, 3},
+    {{ROLE_T_Z, 512, "r8x8x8/E8/G1/split/pre"}, 3},
+    {{ROLE_T_Y_INV, 128, "r8x4x4/E8/G8/split/wide4"}, 3},
+    {{ROLE_T_X_INV, 128, "r8x4x4/E8/G8"}, 3},
+    {{ROLE_T_X_INV, 256, "r8x8x4/E8/G8"}, 3}};
+constexpr CachedVariant kCachedF32[] = {
+    {{ROLE_T_X_FWD, 256, "r16x16/E16/G16/split"}, 6},
+    {{ROLE_T_X_FWD, 512, "r8x8x8/E8/G16/split/wide"}, 6},
+    {{ROLE_T_Y_FWD, 512, "r8x8x8/E8/G16/split"}, 3},
+    {{ROLE_T_Z, 128, "r16x8/E16/G8/split"}, 3},
+    {{ROLE_T_Z, 256, "r8x8x4/E8/G2/split/pre"}, 3},
+    {{ROLE_T_Z, 512, "r8x8x8/E8/G2/split"}, 3},
+    {{ROLE_T_Y_INV, 128, "r16x8/E16/G16/split/wide2"}, 3},
+    {{ROLE_T_X_INV, 512, "r8x8x8/E8/G16"}, 3}};
+constexpr CachedVariant kCachedXp[] = {
+    {{ROLE_T_X_FWD, 256, "r16x16/E16/xp/G16/split/wide"}, 3},
+    {{ROLE_T_X_FWD, 512, "r8x8x8/E8/xp/G16/split/wide"}, 3},
+    {{ROLE_T_X_INV, 256, "r8x8x4/E8/xp/G16"}, 6}};
 
-template <typename T>
-void pick_variants(pfc_hip_plan_s *p, const DefaultVariant *d, size_t count) {
-  for (size_t i = 0; i < count; ++i) {
-    if (p->role_len(d[i].role) != d[i].n) continue;
-    const int nv = variant_count<T>(p, d[i].role);
-    for (int v = 0; v < nv; ++v)
-      if (*variant_name<T>(p, d[i].role, v) == d[i].name) p->var[d[i].role] = v;
-  }
+template <typename T> void pick_variant(pfc_hip_plan_s *p, const DefaultVariant &d) {
+  if (p->role_len(d.role) != d.n) return;
+  const int nv = variant_count<T>(p, d.role);
+  for (int v = 0; v < nv; ++v)
+    if (*variant_name<T>(p, d.role, v) == d.name) p->var[d.role] = v;
 }
 
-// The transposed z pass depends on the model too, which the operators set: the
-// table forms mark their lines non-temporal, which is right where the next pass
-// finds them in HBM anyway and wrong for a PFC run whose three spectra (A2, B2,
-// A1) the 256 MB last-level cache holds.  ms per step of a run, plain lines
-// against the table form: FP32 256^3 .129 / .137, 256x256x128 .076 / .085,
-// 256x128x512 .140 / .145, FP64 256x128x128 .070 / .075; beyond the cache FP32
-// 256x256x512 (3 x 135 MB) .254 / .250.  Tungsten's multipliers cost more than
-// the lines: the table form is ahead at every size (FP64 256x128x128 .141).
-constexpr size_t kLastLevelCache = 256u << 20;
-template <typename T> void default_z(pfc_hip_plan_s *p) {
-  if (p->chosen[ROLE_T_Z] || p->xp || !p->t_ok) return;
-  const bool cached = 3 * p->outbox() * 2 * p->esize <= kLastLevelCache && !p->tungsten();
-  if (cached && sizeof(T) == 8)
-    pick_variants<T>(p, kCachedZF64, std::size(kCachedZF64));
-  else if (cached)
-    pick_variants<T>(p, kCachedZF32, std::size(kCachedZF32));
+template <typename T, typename Pick> void each_default(const pfc_hip_plan_s *p, Pick pick) {
+  if (p->xp)
+    std::for_each(std::begin(kDefaultXp), std::end(kDefaultXp), pick);
+  else if (sizeof(T) == 8)
+    std::for_each(std::begin(kDefaultF64), std::end(kDefaultF64), pick);
   else
-    for (const DefaultVariant &d : kDefaultF64)
-      if (d.role == ROLE_T_Z && sizeof(T) == 8) pick_variants<T>(p, &d, 1);
-  if (!cached && sizeof(T) == 4)
-    for (const DefaultVariant &d : kDefaultF32)
-      if (d.role == ROLE_T_Z) pick_variants<T>(p, &d, 1);
+    std::for_each(std::begin(kDefaultF32), std::end(kDefaultF32), pick);
+}
+
+template <typename T, typename Pick> void each_cached(const pfc_hip_plan_s *p, Pick pick) {
+  if (p->xp)
+    std::for_each(std::begin(kCachedXp), std::end(kCachedXp), pick);
+  else if (sizeof(T) == 8)
+    std::for_each(std::begin(kCachedF64), std::end(kCachedF64), pick);
+  else
+    std::for_each(std::begin(kCachedF32), std::end(kCachedF32), pick);
+}
+
+// The transposed passes depend on the footprint and, through it, on the model,
+// which the operators set: a non-temporal line is right where the next pass finds
+// its grid in HBM anyway and wrong where the last-level cache would hold it.  A PFC
+// run keeps three spectra (A2, B2, A1); us of a single step | a step of a run, both
+// with every other pass as it is here, plain line against non-temporal:
+//   FP64 256x128x128  x fwd 96 / 102 | 71 / 72      x inv 98 / 102 | 71 / 72
+//   FP64 256x256x128  x fwd 182 / 192 | 128 / 128   y fwd 182 / 192 | 124 / 128
+//   FP64 256x128x256  y inv 189 / 195 | 126 / 132   x inv 185 / 195 | 131 / 132
+//   FP32 256x256x128  x fwd 98 / 107 | 77 / 77
+//   FP32 512x128x128  x fwd 99 / 104 | 78 / 79      y inv 104 / 104 | 76 / 79
+//   FP32 1024x128x128 y inv 194 / 207 | 141 / 147   x inv 198 / 207 | 146 / 147
+//   FP32 256x512x128  y fwd 195 / 202 | 138 / 142
+//   FP32 with FP64 butterflies 512x256x128 x fwd 208 / 224
+// and beyond it FP32 512x512x128 x fwd 376 / 359, FP64 256x256x512 y fwd 554 / 533
+// (run).  The FP32 x pass reads a field and writes one spectrum while the previous
+// step's lines leave the cache: plain up to 42 MB, at 67 MB 256^3 191 / 188 and
+// 512x256x128 197 / 188.  z pass, plain lines against the table form, in a run: FP32 256^3
+// 129 / 137, FP64 256x128x128 70 / 75, beyond the cache FP32 256x256x512 254 / 250;
+// of the plain FP32 forms, split against full transposition in a single step
+// 256x256x128 101 / 107, 1024x128x128 195 / 207 (runs equal), and at 256 points
+// tables read ahead 256^3 178 / 188 | 131 / 133.  Tungsten's multipliers cost more
+// than the lines: it keeps the forms of large grids.
+template <typename T> void transposed_defaults(pfc_hip_plan_s *p) {
+  if (!p->t_ok) return;
+  const size_t spectrum = p->outbox() * 2 * p->esize;
+  for (int r : {ROLE_T_X_FWD, ROLE_T_Y_FWD, ROLE_T_Z, ROLE_T_Y_INV, ROLE_T_X_INV}) {
+    if (p->chosen[r]) continue;
+    p->var[r] = 0;
+    each_default<T>(p, [&](const DefaultVariant &d) {
+      if (d.role == r) pick_variant<T>(p, d);
+    });
+    if (p->tungsten()) continue;
+    each_cached<T>(p, [&](const CachedVariant &c) {
+      if (c.d.role == r && c.spectra * spectrum <= kLastLevelCache) pick_variant<T>(p, c.d);
+    });
+  }
 }
 
 // The variant each role of a new plan starts with.
 template <typename T> void default_variants(pfc_hip_plan_s *p) {
-  if (p->xp)
-    pick_variants<T>(p, kDefaultXp, std::size(kDefaultXp));
-  else if (sizeof(T) == 8)
-    pick_variants<T>(p, kDefaultF64, std::size(kDefaultF64));
-  else
-    pick_variants<T>(p, kDefaultF32, std::size(kDefaultF32));
+  each_default<T>(p, [&](const DefaultVariant &d) { pick_variant<T>(p, d); });
+  transposed_defaults<T>(p);
   for (int r = 0; r < ROLE_COUNT; ++r)
     if (plane_role(r) && row_variant_count<T>(p, r) > 0 && plane_variant_default(p))
       p->var[r] = row_variant_count<T>(p, r);
@@ -1454,7 +1502,7 @@ template <typename T> void default_variants(pfc_hip_plan_s *p) {
 // accurate, 7.5e-8 against 9.0e-8, but 8e-8 away).
 template <typename T> void model_variants(pfc_hip_plan_s *p) {
   if (sizeof(T) == 8 || p->xp) {
-    default_z<T>(p);
+    transposed_defaults<T>(p);
     return;
   }
   int kept[ROLE_COUNT];
@@ -1465,7 +1513,6 @@ template <typename T> void model_variants(pfc_hip_plan_s *p) {
     default_variants<T>(p);
   for (int r = 0; r < ROLE_COUNT; ++r)
     if (p->chosen[r] || r == ROLE_STEP_LAYOUT || r == ROLE_STEP_FUSE) p->var[r] = kept[r];
-  if (!p->tungsten()) default_z<T>(p);
 }
 
 int check_plan(pfc_hip_plan_t p) {
